@@ -425,6 +425,17 @@ int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_docs, const f
                   long long s_oh, long long s_on, int P, float scale, int skip, float beta,
                   int top_k, int force, const float* wfix, int nsplit, float* out, float* w,
                   float* r, float* rmax, void* workspace, size_t workspace_bytes, void* stream);
+/* The same read of queries in any layout with hd contiguous (element strides, multiples of 4: qd by
+ * document, row and head, qo by row and head), also writing n [D] fp32 (may be NULL): the keys of
+ * document d that entered r_d, N_d - skip (N_d when N_d <= skip). */
+int xenc_d18_read_strided(int dtype, int T, int hq, int hkv, int hd, int n_docs, const float* qd,
+                          long long s_qd_doc, long long s_qd_row, long long s_qd_head, const float* qo,
+                          long long s_qo_row, long long s_qo_head, const void* k_docs, const void* v_docs,
+                          long long s_dh, long long s_dn, const int* doc_ptr, const float* k_own,
+                          const float* v_own, long long s_oh, long long s_on, int P, float scale, int skip,
+                          float beta, int top_k, int force, const float* wfix, int nsplit, float* out,
+                          float* w, float* r, float* rmax, float* n, void* workspace,
+                          size_t workspace_bytes, void* stream);
 
 /*
  * ---- Calibration (roofline denominators measured on the device; no counterpart in the reference)

@@ -139,6 +139,15 @@ SIGNATURES = {
         c_float, c_int, c_float, c_int, c_int, c_void_p, c_int,  # scale, skip, beta, top_k, force, wfix, nsplit
         c_void_p, c_void_p, c_void_p, c_void_p,      # out, w, r, rmax
         c_void_p, c_size_t, c_void_p]),              # workspace, workspace_bytes, stream
+    "xenc_d18_read_strided": (c_int, [
+        c_int, c_int, c_int, c_int, c_int, c_int,    # dtype, T, hq, hkv, hd, n_docs
+        c_void_p, c_longlong, c_longlong, c_longlong,  # qd, strides (document, row, head)
+        c_void_p, c_longlong, c_longlong,            # qo, strides (row, head)
+        c_void_p, c_void_p, c_longlong, c_longlong, c_void_p,  # k_docs, v_docs, s_dh, s_dn, doc_ptr
+        c_void_p, c_void_p, c_longlong, c_longlong, c_int,     # k_own, v_own, s_oh, s_on, P
+        c_float, c_int, c_float, c_int, c_int, c_void_p, c_int,  # scale, skip, beta, top_k, force, wfix, nsplit
+        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,      # out, w, r, rmax, n
+        c_void_p, c_size_t, c_void_p]),              # workspace, workspace_bytes, stream
     "xenc_gather_pages": (c_int, [
         c_void_p, c_int, c_longlong, c_int,          # pages, slots_per_page, page_stride, d
         c_void_p, c_int, c_int, c_void_p, c_longlong,  # chunk_page, n_chunks, n_flat, idx, ld_idx

@@ -8,7 +8,8 @@
 //   routing:     w = softmax_d(beta * r)  (top_k kept, ties to the lower index; or force / wfix)
 //   output:      o = sum_d w_d o_d                     (before the gate and o_proj)
 //
-// Two launches.  d18_partials_kernel: one workgroup per (row, kv head, unit, key split), the
+// Two launches.  From 16 rows on, d18_tile_kernel and d18_merge_rows_kernel (below); for fewer rows
+// (decode) these two.  d18_partials_kernel: one workgroup per (row, kv head, unit, key split), the
 // units being the D documents and the own rows, each cut into S key ranges so that a few rows
 // (decode) still spread over the GPU; it streams its keys once for all G query heads (GQA) with
 // an online softmax in the log2 domain, and for a document also the max / sum of the keys past
@@ -24,6 +25,7 @@
 // row to arrive on a counter, measured slower: each level adds an L2 write-back, an atomic and
 // two rounds of loads to the critical path.)  Deterministic: every sum runs in a fixed order.
 #include <algorithm>
+#include <cfloat>
 
 #include "xenc_common.h"
 
@@ -119,8 +121,9 @@ __device__ __forceinline__ void wave_sync_lds() {
 struct D18Args {
   int T, hq, hkv, n_docs, S, P, skip, top_k, force;
   float scale_log2, beta;
-  const float* qd;
+  const float* qd;       // element strides: document, row, head (hd contiguous)
   const float* qo;
+  long long s_qdd, s_qdt, s_qdh, s_qot, s_qoh;
   const void* kd;
   const void* vd;
   long long s_dh, s_dn;
@@ -134,6 +137,7 @@ struct D18Args {
   float* w;              // w, r, rmax: [hkv][G][T][D]
   float* r;
   float* rmax;
+  float* n;              // [D] keys that entered r (N_d - skip, or N_d when N_d <= skip); may be NULL
 };
 
 // The query rows of the 16 padded heads in chunks of 8 dims: chunk c = thread + 256 j is head
@@ -141,11 +145,11 @@ struct D18Args {
 // chunks c < HD carry values: a thread loads at most one chunk (HD <= 256), from head
 // min(g, G - 1) so the loads are unconditional; store_q writes heads past G as 0.
 template <int HD>
-__device__ __forceinline__ void load_q(const float* __restrict__ q, int G, f32x4_t (&qv)[2]) {
+__device__ __forceinline__ void load_q(const float* __restrict__ q, long long s_qh, int G, f32x4_t (&qv)[2]) {
   constexpr int CPR = HD / 8;
   const int c = min((int)threadIdx.x, HD - 1);
   const int g = c / CPR, e0 = (c % CPR) * 8;
-  const f32x4_t* src = reinterpret_cast<const f32x4_t*>(q + min(g, G - 1) * HD + e0);
+  const f32x4_t* src = reinterpret_cast<const f32x4_t*>(q + min(g, G - 1) * s_qh + e0);
   qv[0] = src[0];
   qv[1] = src[1];
 }
@@ -204,7 +208,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const TK* base, long
 }
 
 // One key split (n keys, the first at index j_base of its unit; n <= 0: empty) for the G query
-// heads of a kv head (query rows q [G][HD]), hd = HD.  Wave wv takes the 16-key tiles wv, wv + 4,
+// heads of a kv head (query rows q, s_qh elements apart), hd = HD.  Wave wv takes the 16-key tiles wv, wv + 4,
 // ...  The first tile's K and V rows and the query rows are requested together, so the query's
 // latency overlaps the keys'; with 16-bit rows the second tile's rows are requested too.
 // Scores on the matrix cores: S^T [16 keys x 16 heads] = K_tile . Q^T with
@@ -224,7 +228,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const TK* base, long
 template <typename TK, int HD, int GP>
 __device__ __forceinline__ void d18_unit(int G, const TK* __restrict__ K, const TK* __restrict__ V, long long s_n,
                                          int n, int j_base, int skip_c, const float* __restrict__ q,
-                                         float scale_log2, f32x4_t* __restrict__ ml_out,
+                                         long long s_qh, float scale_log2, f32x4_t* __restrict__ ml_out,
                                          float* __restrict__ acc_out, D18Lds& lds) {
   constexpr int EPL = D18Elem<TK>::EPL;
   constexpr int TPR = HD / EPL;              // lanes per row: a power of two <= 64
@@ -459,7 +463,7 @@ __device__ __forceinline__ void d18_unit(int G, const TK* __restrict__ K, const 
     u32x4_t k0[NI], v0[NI], k1[NI], v1[NI];
     load_rows(K, t_first, k0);
     load_rows(V, t_first, v0);
-    load_q<HD>(q, G, qv);
+    load_q<HD>(q, s_qh, G, qv);
     load_rows(K, t_first + kStep, k1);
     load_rows(V, t_first + kStep, v1);
     store_q<TK, HD>(qv, G, scale_log2, lds);
@@ -485,7 +489,7 @@ __device__ __forceinline__ void d18_unit(int G, const TK* __restrict__ K, const 
     u32x4_t kr[NI], vr[NI];
     load_rows(K, t_first, kr);
     load_rows(V, t_first, vr);
-    load_q<HD>(q, G, qv);
+    load_q<HD>(q, s_qh, G, qv);
     store_q<TK, HD>(qv, G, scale_log2, lds);
     __syncthreads();
     for (int t0 = t_first; t0 < n; t0 += kStep) {
@@ -608,6 +612,12 @@ __device__ __forceinline__ float doc_weight(float r, bool has, int d, int D, flo
   return e / wave_sum(e);
 }
 
+// The keys of document d that enter r: those past `skip`, or all when there are no more than skip.
+__device__ __forceinline__ float counted_keys(const int* __restrict__ doc_ptr, int d, int skip) {
+  const int N = doc_ptr[d + 1] - doc_ptr[d];
+  return (float)(N > skip ? N - skip : N);
+}
+
 // One workgroup of 2 waves per (row t, kv head h, query head g) and block of 16 output dims:
 // blockIdx.x = (t * hkv + h) * G + g, blockIdx.y = dim block.  Each 16-lane row of the
 // workgroup merges one unit (row k of the 8 takes units k, k + 8, ...): lane j of the row holds
@@ -622,7 +632,8 @@ constexpr int kD18MergeDims = 16;
 constexpr int kD18MergeThreads = 128;
 constexpr int kD18MergeRows = kD18MergeThreads / kD18MergeDims;   // units in flight
 
-__global__ __launch_bounds__(kD18MergeThreads) void d18_merge_kernel(const D18Args A, int hd) {
+__global__ __launch_bounds__(kD18MergeThreads) void d18_merge_kernel(const D18Args A, int hd,
+                                                                     const int* __restrict__ doc_ptr) {
   __shared__ f32x4_t ust[kD18MaxDocs + 1];                 // per unit: (M, L, Mc, Lc)
   __shared__ float ua[kD18MaxDocs + 1][kD18MergeDims];     // per unit: the merged accumulator
   __shared__ float wl[kD18MaxDocs];
@@ -659,6 +670,7 @@ __global__ __launch_bounds__(kD18MergeThreads) void d18_merge_kernel(const D18Ar
   {
     const int d = lane;
     const bool has = d < D;
+    if (A.n && blockIdx.x == 0 && blockIdx.y == 0 && has) A.n[d] = counted_keys(doc_ptr, d, A.skip);
     const f32x4_t st = has ? ust[d] : empty;
     const float r = st[3] > 0.f ? st[2] * kLn2 + logf(st[3]) : -INFINITY;
     const float w = doc_weight(r, has, d, D, A.beta, A.top_k, A.force, A.wfix);
@@ -706,17 +718,539 @@ __global__ __launch_bounds__(kD18Threads) void d18_partials_kernel(const D18Args
     const int lo = sp * chunk, n = min(N - lo, chunk);
     const long long off = (long long)h * A.s_dh + (long long)(n0 + lo) * A.s_dn;
     d18_unit<TD, HD, GP>(G, static_cast<const TD*>(A.kd) + off, static_cast<const TD*>(A.vd) + off, A.s_dn, n, lo,
-                         N > A.skip ? A.skip : 0, A.qd + (((long long)u * A.T + t) * A.hq + (long long)h * G) * HD,
-                         A.scale_log2, A.part_ml + slot, A.part_acc + slot * HD, lds);
+                         N > A.skip ? A.skip : 0,
+                         A.qd + u * A.s_qdd + t * A.s_qdt + (long long)h * G * A.s_qdh, A.s_qdh, A.scale_log2, A.part_ml + slot, A.part_acc + slot * HD, lds);
   } else {
     const int chunk = (A.P + A.T + A.S - 1) / A.S;
     const int lo = sp * chunk, n = min(A.P + t + 1 - lo, chunk);
     const long long off = (long long)h * A.s_oh + (long long)lo * A.s_on;
     d18_unit<float, HD, GP>(G, A.ko + off, A.vo + off, A.s_on, n, lo, -1,
-                            A.qo + ((long long)t * A.hq + (long long)h * G) * HD, A.scale_log2, A.part_ml + slot,
-                            A.part_acc + slot * HD, lds);
+                            A.qo + t * A.s_qot + (long long)h * G * A.s_qoh, A.s_qoh, A.scale_log2,
+                            A.part_ml + slot, A.part_acc + slot * HD, lds);
   }
 }
+
+// ------------------------------------------------------------------------------------------
+// Many rows.  d18_tile_kernel: one workgroup of 4 waves per (64 columns, kv head, unit, key split),
+// a column being one (row t, query head g) of the kv head (column t * G + g); wave wv holds columns
+// 16 wv .. + 15 with its query parts in registers, and every wave reads the same key / value
+// tiles from LDS, so a key row is fetched once per 64 columns instead of once per reader row.
+// Same products and the same fp32-accurate splits as d18_unit; lane (k4 = lane / 16, hs = lane % 16)
+// holds column hs and, of each 16-key score tile, keys 4 k4 + r.  Those scores are the A operand
+// of P.V as they stand (k slot 8 k4 + e <-> key 4 k4 + e of the first 16 keys, e < 4, and of the
+// second, e >= 4): 16-bit values take 32 keys per MFMA and part of p, with no padding slots; fp32
+// values run on v_mfma_f32_16x16x4_f32 (k slot k4 <-> key 4 k4 + r), whole fp32 products.
+// Tiles go from global memory straight to LDS, two stages, one barrier a tile.  A row's 16-byte
+// chunk c sits at position c ^ (row & 15): the 16-byte key reads (8 rows at one chunk) and the
+// 4-byte value reads (rows r, 4 + r, 8 + r, 12 + r at one 64-byte group) then fall on disjoint banks.
+__device__ __forceinline__ uint2 lds_read_tr16(const char* p) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(
+      uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(uintptr_t)(const __attribute__((address_space(3))) char*)p));
+}
+
+constexpr int kTileThreads = 256;
+constexpr int kTileCols = 64;
+constexpr int kTileStage = 32 * 1024;   // K and V of a tile: 32 16-bit or 16 fp32 rows of 256 dims
+
+template <typename TK, int HD>
+__device__ __forceinline__ void d18_tile_unit(const TK* __restrict__ K, const TK* __restrict__ V, long long s_n, int n,
+                                              int lim, int j_base, int skip_c, const float* __restrict__ q,
+                                              bool live, float scale_log2, const D18Args& A, long long slot_h,
+                                              int ct, char* __restrict__ lds) {
+  constexpr bool kF32 = sizeof(TK) == 4, kBf16 = __is_same(TK, __bf16);
+  constexpr int EPC = 16 / (int)sizeof(TK), CPR = HD / EPC;   // elements per chunk, chunks per row
+  constexpr int KT = kF32 ? 16 : 32, NT = KT / 16;            // keys, score tiles per staged tile
+  constexpr int XM = (CPR < 16 ? CPR : 16) - 1;
+  constexpr int NLD = 2 * KT * CPR / kTileThreads;            // staged chunks per thread
+  constexpr int KB = HD / 32, NP = kBf16 ? 3 : 2, ROWB = HD * (int)sizeof(TK);
+  static_assert(2 * KT * ROWB <= kTileStage && NLD >= 1, "a staged tile");
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int hs = lane % 16, k4 = lane / 16;
+  const bool hi16 = (lane & 16) != 0, hi32 = (lane & 32) != 0;
+  const int G = A.hq / A.hkv;
+
+  // Stage the K and V rows t0 .. t0 + KT - 1 (past the split: its last row again; masked).
+  auto issue = [&](int st, int t0) {
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const int w0 = i * kTileThreads + wv * kWave;   // first chunk of this wave's load
+      const bool isv = w0 >= KT * CPR;                // wave-uniform
+      const int id = w0 + lane - (isv ? KT * CPR : 0);
+      const int row = id / CPR, c = (id % CPR) ^ (row & XM);
+      const TK* src = (isv ? V : K) + (long long)min(t0 + row, n - 1) * s_n + c * EPC;
+      stage_to_lds(lds + st * kTileStage + w0 * 16, src);
+    }
+  };
+  if (n > 0) issue(0, 0);
+
+  // This lane's column of the query in parts (see store_q): dims 32 kb + 8 k4 .. + 7.
+  u32x4_t qp[NP][KB];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    f32x4_t x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
+    if (live) {
+      x0 = *reinterpret_cast<const f32x4_t*>(q + 32 * kb + 8 * k4);
+      x1 = *reinterpret_cast<const f32x4_t*>(q + 32 * kb + 8 * k4 + 4);
+    }
+    unsigned short h[NP][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = (e < 4 ? x0[e % 4] : x1[e % 4]) * scale_log2;
+      if constexpr (kBf16) {
+        const __bf16 p0 = (__bf16)x;
+        const float r1 = x - (float)p0;
+        const __bf16 p1 = (__bf16)r1;
+        h[0][e] = __builtin_bit_cast(unsigned short, p0);
+        h[1][e] = __builtin_bit_cast(unsigned short, p1);
+        h[2][e] = __builtin_bit_cast(unsigned short, (__bf16)(r1 - (float)p1));
+      } else {
+        h[0][e] = __builtin_bit_cast(unsigned short, f16_hi(x));
+        h[1][e] = __builtin_bit_cast(unsigned short, f16_lo(x));
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) qp[p][kb][i] = (unsigned)h[p][2 * i] | ((unsigned)h[p][2 * i + 1] << 16);
+  }
+
+  f32x4_t acc[HD / 16];   // columns 4 k4 + r, dim 16 b + hs
+#pragma unroll
+  for (int b = 0; b < HD / 16; ++b) acc[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f, mc = -INFINITY, lc = 0.f, mt = -INFINITY;   // column hs
+  const int cmode = skip_c < 0 || j_base + n <= skip_c ? 0 : j_base >= skip_c ? 1 : 2;   // see d18_unit
+  // The least key limit of the wave's live columns (own rows are causal: the limits differ by row).
+  const int lim_min = -(int)wave_max(live ? (float)-lim : -1e9f);
+  const bool any_live = __ballot(live) != 0;   // wave-uniform
+
+  // LDS byte offsets in a stage.  Chunk 4 c + a of row `row` (a < 4) is at row * ROWB + 16 ((4 c + a)
+  // ^ (row & XM)) = (row * ROWB + 16 (a ^ (row & XM))) ^ 64 c, rows being powers of two.
+  const int k_off = hs * ROWB + (((kF32 ? 2 * k4 : k4) ^ (hs & XM)) << 4);
+  // fp32 values: word hs of row 4 k4 + r, the 4-byte B operand.  16-bit values: the 8 bytes that
+  // lane (k4, hs) supplies to ds_read_b64_tr_b16, dims 4 (hs % 4) .. + 3 of row 4 k4 + hs / 4: the
+  // transposing read returns dim hs of rows 4 k4 .. + 3 (the 16 lanes of a row group exchange).
+  constexpr int NVO = kF32 ? 4 : 1;
+  int v_off[NVO];
+#pragma unroll
+  for (int r = 0; r < NVO; ++r) {
+    const int row = 4 * k4 + (kF32 ? r : hs / 4);
+    v_off[r] = (KT + row) * ROWB + (((kF32 ? hs / 4 : hs % 4 / 2) ^ (row & XM)) << 4) +
+               (kF32 ? hs % 4 * 4 : hs % 2 * 8);
+  }
+
+  auto tile = [&](int stage, int t0) {
+    // (opaque per tile: left alone, the compiler keeps every XORed offset in a register of its own)
+    int ko = k_off + stage, vo[NVO];
+    asm volatile("" : "+v"(ko));
+#pragma unroll
+    for (int r = 0; r < NVO; ++r) {
+      vo[r] = v_off[r] + stage;
+      asm volatile("" : "+v"(vo[r]));
+    }
+    f32x4_t sc[NT];
+    {
+      f32x4_t s[NT][3];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) s[t][p] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      // The key fragments of k step kb + 1 are read while the products of step kb issue; the scheduling
+      // barriers hold that order (left alone, every read lands right before its use).
+      constexpr int KC = kF32 ? 2 : 1;   // 16-byte chunks of a fragment
+      u32x4_t kf[2][NT][KC];
+      auto read_k = [&](int kb) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int c = 0; c < KC; ++c)
+            kf[kb % 2][t][c] = *reinterpret_cast<const u32x4_t*>(lds + 16 * t * ROWB + ((ko ^ (64 * KC * kb)) ^ (16 * c)));
+      };
+      read_k(0);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        if (kb + 1 < KB) {
+          read_k(kb + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const u32x4_t* f = kf[kb % 2][t];
+          if constexpr (kBf16) {
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+              s[t][p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  __builtin_bit_cast(d18_bf8, f[0]), __builtin_bit_cast(d18_bf8, qp[p][kb]), s[t][p], 0, 0, 0);
+          } else {
+            const d18_half8 qh = __builtin_bit_cast(d18_half8, qp[0][kb]), ql = __builtin_bit_cast(d18_half8, qp[1][kb]);
+            if constexpr (kF32) {
+              d18_half8 ka, kl;
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                const float x = __uint_as_float(f[e / 4][e % 4]);
+                ka[e] = f16_hi(x);
+                kl[e] = f16_lo(x);
+              }
+              s[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh, s[t][0], 0, 0, 0);
+              s[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql, s[t][1], 0, 0, 0);
+              s[t][2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh, s[t][2], 0, 0, 0);
+            } else {
+              const d18_half8 ka = __builtin_bit_cast(d18_half8, f[0]);
+              s[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh, s[t][0], 0, 0, 0);
+              s[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql, s[t][1], 0, 0, 0);
+            }
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) sc[t] = (s[t][0] + s[t][1]) + s[t][2];
+    }
+    // Online softmax of column hs over keys t0 + 16 t + 4 k4 + r (as d18_unit's).
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (t0 + 16 * t + 4 * k4 + r < lim) mx = fmaxf(mx, sc[t][r]);
+    mx = fmaxf(mx, swap_partner<16>(mx, hi16));
+    mx = fmaxf(mx, swap_partner<32>(mx, hi32));
+    const float mn = mx > m + kD18Lazy ? mx : m;
+    mt = fmaxf(mt, mx);
+    const float a = rescale(m, mn);
+    const bool any_rescale = __ballot(m != -INFINITY && mn != m) != 0;   // wave-uniform
+    float pr[NT][4], ps = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pr[t][r] = t0 + 16 * t + 4 * k4 + r < lim ? __builtin_amdgcn_exp2f(sc[t][r] - mn) : 0.f;
+        ps += pr[t][r];
+      }
+    ps += swap_partner<16>(ps, hi16);
+    ps += swap_partner<32>(ps, hi32);
+    l = l * a + ps;
+    m = mn;
+    if (cmode == 2) {
+      float mcx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int k = t0 + 16 * t + 4 * k4 + r;
+          if (k < lim && j_base + k >= skip_c) mcx = fmaxf(mcx, sc[t][r]);
+        }
+      mcx = fmaxf(mcx, swap_partner<16>(mcx, hi16));
+      mcx = fmaxf(mcx, swap_partner<32>(mcx, hi32));
+      const float mcn = fmaxf(mc, mcx);
+      float cs = 0.f;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int k = t0 + 16 * t + 4 * k4 + r;
+          if (k < lim && j_base + k >= skip_c) cs += __builtin_amdgcn_exp2f(sc[t][r] - mcn);
+        }
+      cs += swap_partner<16>(cs, hi16);
+      cs += swap_partner<32>(cs, hi32);
+      lc = lc * rescale(mc, mcn) + cs;
+      mc = mcn;
+    }
+    if (any_rescale) {
+      float al[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) al[r] = __shfl(a, 4 * k4 + r);
+#pragma unroll
+      for (int b = 0; b < HD / 16; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[b][r] *= al[r];
+    }
+    if constexpr (!kF32) {
+      u32x4_t ap[NP];   // p in 16-bit parts: bf16 hi, mid, lo (24 bits), fp16 hi, lo (22 bits)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        unsigned short h[NP][4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if constexpr (kBf16) {
+            const __bf16 p0 = (__bf16)pr[t][r];
+            const float r1 = pr[t][r] - (float)p0;
+            const __bf16 p1 = (__bf16)r1;
+            h[0][r] = __builtin_bit_cast(unsigned short, p0);
+            h[1][r] = __builtin_bit_cast(unsigned short, p1);
+            h[2][r] = __builtin_bit_cast(unsigned short, (__bf16)(r1 - (float)p1));
+          } else {
+            h[0][r] = __builtin_bit_cast(unsigned short, f16_hi(pr[t][r]));
+            h[1][r] = __builtin_bit_cast(unsigned short, f16_lo(pr[t][r]));
+          }
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+          ap[p][2 * t] = (unsigned)h[p][0] | ((unsigned)h[p][1] << 16);
+          ap[p][2 * t + 1] = (unsigned)h[p][2] | ((unsigned)h[p][3] << 16);
+        }
+      }
+      // Pairs of 16-dim blocks; the next pair's values are read while this pair's products issue.
+      u32x4_t bv[2][2];   // [pair % 2][block]: dim 16 b + hs of the 8 key slots
+      auto read_v = [&](int c) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            const uint2 w = lds_read_tr16(lds + 16 * t * ROWB + (vo[0] ^ (32 * (2 * c + j))));
+            bv[c % 2][j][2 * t] = w.x;
+            bv[c % 2][j][2 * t + 1] = w.y;
+          }
+      };
+      read_v(0);
+#pragma unroll
+      for (int c = 0; c < HD / 32; ++c) {
+        if (c + 1 < HD / 32) {
+          read_v(c + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // (the tile's sum is formed from 0 and added once: three parts rounding against the running
+        // sum of a long split cost 5e-7 of the result against 3.4e-7 this way, and 3 % of time)
+        f32x4_t x[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int p = NP - 1; p >= 0; --p)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            if constexpr (kBf16)
+              x[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(d18_bf8, ap[p]),
+                                                             __builtin_bit_cast(d18_bf8, bv[c % 2][j]), x[j], 0, 0, 0);
+            else
+              x[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(d18_half8, ap[p]),
+                                                            __builtin_bit_cast(d18_half8, bv[c % 2][j]), x[j], 0, 0, 0);
+          }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[2 * c + j] += x[j];
+      }
+    } else {
+      // A key that some columns see and others do not (own rows, causal) enters the product with
+      // p = 0 for the others: a non-finite value there must not reach them (0 * inf), so it is left
+      // out of the product and added below to the columns that see it.
+      const bool diag = t0 + KT > lim_min;
+      bool bad = false;
+      constexpr int NB = HD / 16 < 4 ? HD / 16 : 4;   // 16-dim blocks per step
+      float fv[2][4][NB];
+      auto read_v = [&](int i) {   // keys 4 k4 + r, blocks NB i .. + NB - 1
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < NB; ++j)
+            fv[i % 2][r][j] = *reinterpret_cast<const float*>(lds + (vo[r] ^ (64 * (NB * i + j))));
+      };
+      read_v(0);
+#pragma unroll
+      for (int i = 0; i < HD / 16 / NB; ++i) {
+        if (i + 1 < HD / 16 / NB) {
+          read_v(i + 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        f32x4_t x[NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) x[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const bool some = diag && t0 + 4 * k4 + r >= lim_min;
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            const float v = fv[i % 2][r][j];
+            const bool out = some && !(fabsf(v) <= FLT_MAX);
+            bad |= out;
+            x[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pr[0][r], out ? 0.f : v, x[j], 0, 0, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[NB * i + j] += x[j];
+      }
+      if (__ballot(bad) != 0) {
+#pragma unroll 1
+        for (int kq = 0; kq < 4; ++kq)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int kk = 4 * kq + r;
+            if (t0 + kk < lim_min || t0 + kk >= n) continue;   // wave-uniform
+            float pc[4];   // p of key kk for columns 4 k4 + rr, and whether they see it
+            bool sees[4];
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+              pc[rr] = __shfl(pr[0][r], kq * 16 + 4 * k4 + rr);
+              sees[rr] = t0 + kk < __shfl(lim, 4 * k4 + rr);
+            }
+            const char* vrow = lds + stage + (KT + kk) * ROWB + (hs % 4) * 4;
+#pragma unroll
+            for (int b = 0; b < HD / 16; ++b) {
+              const float v = *reinterpret_cast<const float*>(vrow + (((4 * b + hs / 4) ^ (kk & XM)) << 4));
+              const bool out = !(fabsf(v) <= FLT_MAX);
+#pragma unroll
+              for (int rr = 0; rr < 4; ++rr) acc[b][rr] += out && sees[rr] ? pc[rr] * v : 0.f;
+            }
+          }
+      }
+    }
+  };
+
+  for (int t0 = 0, it = 0; t0 < n; t0 += KT, ++it) {
+    wait_vmem<0>();
+    __syncthreads();   // tile `it` staged by every wave; the other stage is read out
+    if (t0 + KT < n) issue((it + 1) & 1, t0 + KT);
+    if (any_live) tile((it & 1) * kTileStage, t0);
+  }
+  if (cmode == 1) {
+    mc = mt;
+    lc = l * rescale(m, mt);
+  }
+  const int ncol = A.T * G;
+  const long long s_t = (long long)A.hkv * (A.n_docs + 1) * A.S * G;   // part_ml slots per row t
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int c = ct * kTileCols + wv * 16 + 4 * k4 + r;
+    if (c < ncol) {
+      float* o = A.part_acc + (slot_h + (c / G) * s_t + c % G) * HD;
+#pragma unroll
+      for (int b = 0; b < HD / 16; ++b) o[16 * b + hs] = acc[b][r];
+    }
+  }
+  if (k4 == 0 && live) {
+    const int c = ct * kTileCols + wv * 16 + hs;
+    A.part_ml[slot_h + (c / G) * s_t + c % G] = f32x4_t{m, l, mc, lc};
+  }
+}
+
+// Block order: the column tiles of one (split, document, kv head) next to each other on one XCD, so
+// its L2 serves the keys to all but the first; the own rows' workgroups, mostly short, after all of
+// the documents' and dealt over the XCDs (in the documents' order they landed on one or two XCDs, and
+// the others took their share of the documents: 80 against 71 us at the size below).
+// Bound by the matrix pipes with one tile's latencies in between: 130 rows x 16 heads over 4
+// documents of 1000-1500 rows, hd 256 bf16: 243 us with a workgroup per reader row, 60 us here (3
+// splits).  The call: 332 -> 64 us.
+template <typename TD, int HD>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2))) void d18_tile_kernel(
+    const D18Args A, const int* __restrict__ doc_ptr, int col_tiles) {
+  __shared__ alignas(16) char lds[2 * kTileStage];
+  const int G = A.hq / A.hkv, U = A.n_docs + 1;
+  const int n_doc = col_tiles * A.S * A.n_docs * A.hkv;   // the documents' workgroups
+  const bool own = (int)blockIdx.x >= n_doc;
+  int b = own ? (int)blockIdx.x - n_doc : xcd_remap(blockIdx.x, n_doc);
+  const int ct = b % col_tiles;
+  b /= col_tiles;
+  const int sp = b % A.S;
+  b /= A.S;
+  const int u = own ? A.n_docs : b % A.n_docs, h = own ? b : b / A.n_docs;
+  const int c = ct * kTileCols + (threadIdx.x / kWave) * 16 + threadIdx.x % 16;
+  const bool live = c < A.T * G;
+  const int t = live ? c / G : 0, hq = h * G + (live ? c % G : 0);
+  const long long slot_h = (((long long)h * U + u) * A.S + sp) * G;
+  if (u < A.n_docs) {
+    const int n0 = doc_ptr[u], N = doc_ptr[u + 1] - n0;
+    const int chunk = (N + A.S - 1) / A.S;
+    const int lo = sp * chunk, n = min(N - lo, chunk);
+    const long long off = (long long)h * A.s_dh + (long long)(n0 + lo) * A.s_dn;
+    d18_tile_unit<TD, HD>(static_cast<const TD*>(A.kd) + off, static_cast<const TD*>(A.vd) + off, A.s_dn, n, n, lo,
+                          N > A.skip ? A.skip : 0, A.qd + u * A.s_qdd + t * A.s_qdt + hq * A.s_qdh, live, A.scale_log2,
+                          A, slot_h, ct, lds);
+  } else {
+    const int chunk = (A.P + A.T + A.S - 1) / A.S;
+    const int lo = sp * chunk;
+    const int t_last = min(A.T - 1, (ct * kTileCols + kTileCols - 1) / G);
+    const int n = min(A.P + t_last + 1 - lo, chunk);
+    const long long off = (long long)h * A.s_oh + (long long)lo * A.s_on;
+    d18_tile_unit<float, HD>(A.ko + off, A.vo + off, A.s_on, n, min(A.P + t + 1 - lo, chunk), lo, -1,
+                             A.qo + t * A.s_qot + hq * A.s_qoh, live, A.scale_log2, A, slot_h, ct, lds);
+  }
+}
+
+// The merge for many rows: one wave per (row t, query head), lane l holding VEC = hd / 64 (at least 1)
+// output dims; the units' states and weights as in d18_merge_kernel (lane u: unit u), then the
+// accumulators of the splits streamed once, in the same order.  Bound by that stream: 2080 outputs x
+// 15 partials of 1 KB in 12 us (d18_merge_kernel, 16 workgroups an output: 56 us over 5 partials).
+constexpr int kRowsMergeWaves = 4;
+template <int VEC>
+__global__ __launch_bounds__(kRowsMergeWaves * kWave) void d18_merge_rows_kernel(const D18Args A, int hd,
+                                                                                 const int* __restrict__ doc_ptr) {
+  typedef float vec_t __attribute__((ext_vector_type(VEC)));
+  __shared__ f32x4_t ust[kRowsMergeWaves][kD18MaxDocs + 1];
+  __shared__ float wl[kRowsMergeWaves][kD18MaxDocs];
+  const int G = A.hq / A.hkv, U = A.n_docs + 1, D = A.n_docs, S = A.S;
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const int i = blockIdx.x * kRowsMergeWaves + wv;   // wave-uniform
+  if (i >= A.T * A.hq) return;
+  const int t = i / A.hq, hg = i % A.hq, h = hg / G, g = hg % G;
+  const long long slot0 = ((long long)t * A.hkv + h) * U * S * G + g;   // unit u, split s at + (u S + s) G
+  for (int u = lane; u < U; u += kWave) {
+    float M = -INFINITY, Mc = -INFINITY, L = 0.f, Lc = 0.f;
+    for (int s = 0; s < S; ++s) {
+      const f32x4_t st = A.part_ml[slot0 + ((long long)u * S + s) * G];
+      M = fmaxf(M, st[0]);
+      Mc = fmaxf(Mc, st[2]);
+    }
+    for (int s = 0; s < S; ++s) {
+      const f32x4_t st = A.part_ml[slot0 + ((long long)u * S + s) * G];
+      L += st[1] * rescale(st[0], M);
+      Lc += st[3] * rescale(st[2], Mc);
+    }
+    ust[wv][u] = f32x4_t{M, L, Mc, Lc};
+  }
+  wave_sync_lds();
+  {
+    const int d = lane;
+    const bool has = d < D;
+    if (A.n && i == 0 && has) A.n[d] = counted_keys(doc_ptr, d, A.skip);
+    const f32x4_t st = has ? ust[wv][d] : f32x4_t{-INFINITY, 0.f, -INFINITY, 0.f};
+    const float r = st[3] > 0.f ? st[2] * kLn2 + logf(st[3]) : -INFINITY;
+    const float w = doc_weight(r, has, d, D, A.beta, A.top_k, A.force, A.wfix);
+    if (has) {
+      const long long o = ((long long)hg * A.T + t) * D + d;
+      A.w[o] = w;
+      A.r[o] = r;
+      A.rmax[o] = st[3] > 0.f ? st[2] * kLn2 : -INFINITY;
+      wl[wv][d] = w;
+    }
+  }
+  wave_sync_lds();
+  const int e = min(lane * VEC, hd - VEC);   // lanes past hd load valid dims and store nothing
+  auto unit_acc = [&](int u) {
+    const float M = ust[wv][u][0];
+    vec_t a = 0.f;
+#pragma unroll 4
+    for (int s = 0; s < S; ++s) {
+      const long long sl = slot0 + ((long long)u * S + s) * G;
+      const float f = rescale(A.part_ml[sl][0], M);
+      const vec_t v = *reinterpret_cast<const vec_t*>(A.part_acc + sl * hd + e);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) a[j] = fmaf(v[j], f, a[j]);
+    }
+    return a;
+  };
+  const vec_t ao = unit_acc(D);
+  const f32x4_t so = ust[wv][D];
+  vec_t o = 0.f;
+#pragma unroll 2
+  for (int d = 0; d < D; ++d) {
+    const vec_t ad = unit_acc(d);
+    const f32x4_t sd = ust[wv][d];
+    const float M = fmaxf(sd[0], so[0]);
+    const float a = rescale(sd[0], M), b = rescale(so[0], M), den = sd[1] * a + so[1] * b;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) o[j] = fmaf(wl[wv][d], (ad[j] * a + ao[j] * b) / den, o[j]);
+  }
+  if (lane * VEC < hd) *reinterpret_cast<vec_t*>(A.out + ((long long)t * A.hq + hg) * hd + e) = o;
+}
+
+// Rows from which a call takes the tile kernel.  The per-row kernel reads every key again for each
+// row, the tile kernel has the longer chain per workgroup.  Per call, 4 documents of 1500 rows, 2 kv
+// heads, per-row against tile: 8 rows 33 / 37 us (bf16, G 8, hd 256) and 28 / 41 (fp32, G 4, hd 128);
+// 16 rows 47 / 40 (bf16) and 27 / 27 (fp16, G 1, hd 128: the host's share); 32 rows 80 / 46, 39 / 27
+// and 55 / 43 (fp32).
+constexpr int kTileMinRows = 16;
+// Outputs (rows x query heads) from which one wave per output merges: below, d18_merge_kernel's hd / 16
+// workgroups per output are what fills the CUs.
+constexpr int kRowsMergeMin = 256;
 
 size_t d18_align256(size_t x) { return (x + 255) & ~size_t(255); }
 
@@ -731,12 +1265,13 @@ extern "C" size_t xenc_d18_workspace_bytes(int T, int hq, int n_docs, int hd, in
   return d18_align256(units * sizeof(f32x4_t)) + d18_align256(units * hd * sizeof(float));
 }
 
-extern "C" int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_docs, const float* qd,
-                             const float* qo, const void* k_docs, const void* v_docs, long long s_dh,
-                             long long s_dn, const int* doc_ptr, const float* k_own, const float* v_own,
-                             long long s_oh, long long s_on, int P, float scale, int skip, float beta,
-                             int top_k, int force, const float* wfix, int nsplit, float* out, float* w,
-                             float* r, float* rmax, void* workspace, size_t workspace_bytes, void* stream) {
+extern "C" int xenc_d18_read_strided(
+    int dtype, int T, int hq, int hkv, int hd, int n_docs, const float* qd, long long s_qd_doc, long long s_qd_row,
+    long long s_qd_head, const float* qo, long long s_qo_row, long long s_qo_head, const void* k_docs,
+    const void* v_docs, long long s_dh, long long s_dn, const int* doc_ptr, const float* k_own, const float* v_own,
+    long long s_oh, long long s_on, int P, float scale, int skip, float beta, int top_k, int force, const float* wfix,
+    int nsplit, float* out, float* w, float* r, float* rmax, float* n, void* workspace, size_t workspace_bytes,
+    void* stream) {
   if (dtype < 0 || dtype > 2) return XENC_EINVAL;
   if (T < 0 || P < 0 || skip < 0 || top_k < 0 || hkv <= 0 || hq <= 0 || hq % hkv != 0) return XENC_EINVAL;
   if (hq / hkv > kD18MaxG || n_docs < 1 || n_docs > kD18MaxDocs || force >= n_docs || force < -1)
@@ -747,6 +1282,7 @@ extern "C" int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_do
   if (hd != 32 && hd != 64 && hd != 128 && hd != 256) return XENC_EINVAL;
   const int epl = dtype == 2 ? 4 : 8;
   if (s_dh % epl || s_dn % epl || s_oh % 4 || s_on % 4 || s_dn < hd || s_on < hd) return XENC_EALIGN;
+  if (s_qd_doc % 4 || s_qd_row % 4 || s_qd_head % 4 || s_qo_row % 4 || s_qo_head % 4) return XENC_EALIGN;
   if (T == 0) return XENC_OK;
   if (!qd || !qo || !k_docs || !v_docs || !doc_ptr || !k_own || !v_own || !out || !w || !r || !rmax)
     return XENC_ENULL;
@@ -756,7 +1292,7 @@ extern "C" int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_do
   if (!workspace) return XENC_ENULL;
   if (!aligned16(workspace)) return XENC_EALIGN;
   if (workspace_bytes < xenc_d18_workspace_bytes(T, hq, n_docs, hd, nsplit)) return XENC_EWORKSPACE;
-  if ((long long)T * hkv > 0x7fffffffLL) return XENC_EINVAL;
+  if ((long long)T * hq > 0x7fffffffLL) return XENC_EINVAL;
   // A 16-row tile's bytes fit the 32-bit buffer descriptor.
   const long long esz = dtype == 2 ? 4 : 2;
   if ((15 * s_dn + hd) * esz > 0x7fffffffLL || (15 * s_on + hd) * 4 > 0x7fffffffLL) return XENC_EINVAL;
@@ -776,6 +1312,11 @@ extern "C" int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_do
   A.beta = beta;
   A.qd = qd;
   A.qo = qo;
+  A.s_qdd = s_qd_doc;
+  A.s_qdt = s_qd_row;
+  A.s_qdh = s_qd_head;
+  A.s_qot = s_qo_row;
+  A.s_qoh = s_qo_head;
   A.kd = k_docs;
   A.vd = v_docs;
   A.s_dh = s_dh;
@@ -791,10 +1332,32 @@ extern "C" int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_do
   A.w = w;
   A.r = r;
   A.rmax = rmax;
+  A.n = n;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const int G = hq / hkv;
+  if (T >= kTileMinRows) {
+    const int col_tiles = (T * G + kTileCols - 1) / kTileCols;
+    const dim3 tgrid((unsigned)((long long)col_tiles * hkv * (n_docs + 1) * nsplit));
+#define XENC_D18_TILE(TD, HDV) \
+  hipLaunchKernelGGL((d18_tile_kernel<TD, HDV>), tgrid, dim3(kTileThreads), 0, st, A, doc_ptr, col_tiles)
+#define XENC_D18_TILE_HD(TD)                    \
+  switch (hd) {                                 \
+    case 32: XENC_D18_TILE(TD, 32); break;      \
+    case 64: XENC_D18_TILE(TD, 64); break;      \
+    case 128: XENC_D18_TILE(TD, 128); break;    \
+    default: XENC_D18_TILE(TD, 256); break;     \
+  }
+    switch (dtype) {
+      case 0: XENC_D18_TILE_HD(_Float16) break;
+      case 1: XENC_D18_TILE_HD(__bf16) break;
+      default: XENC_D18_TILE_HD(float) break;
+    }
+#undef XENC_D18_TILE_HD
+#undef XENC_D18_TILE
+  } else {
   const dim3 grid((unsigned)(T * hkv), (unsigned)((n_docs + 1) * nsplit));
   // Query heads per kv head padded to 1, 2, 4 or 8 (padded heads have q = 0 and are not written).
-  const int G = hq / hkv, GP = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
+  const int GP = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
 #define XENC_D18_LAUNCH(TD, HDV, GPV) \
   hipLaunchKernelGGL((d18_partials_kernel<TD, HDV, GPV>), grid, dim3(kD18Threads), 0, st, A, doc_ptr)
 #define XENC_D18_GP(TD, HDV)                            \
@@ -819,7 +1382,28 @@ extern "C" int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_do
 #undef XENC_D18_HD
 #undef XENC_D18_GP
 #undef XENC_D18_LAUNCH
-  hipLaunchKernelGGL(d18_merge_kernel, dim3((unsigned)(T * hq), (unsigned)((hd + kD18MergeDims - 1) / kD18MergeDims)),
-                     dim3(kD18MergeThreads), 0, st, A, hd);
+  }
+  if (int rc = check_launch()) return rc;
+  if (T * hq >= kRowsMergeMin) {
+    const dim3 mgrid((unsigned)((T * hq + kRowsMergeWaves - 1) / kRowsMergeWaves)), mblock(kRowsMergeWaves * kWave);
+    if (hd == 256) hipLaunchKernelGGL(d18_merge_rows_kernel<4>, mgrid, mblock, 0, st, A, hd, doc_ptr);
+    else if (hd == 128) hipLaunchKernelGGL(d18_merge_rows_kernel<2>, mgrid, mblock, 0, st, A, hd, doc_ptr);
+    else hipLaunchKernelGGL(d18_merge_rows_kernel<1>, mgrid, mblock, 0, st, A, hd, doc_ptr);
+  } else {
+    hipLaunchKernelGGL(d18_merge_kernel, dim3((unsigned)(T * hq), (unsigned)((hd + kD18MergeDims - 1) / kD18MergeDims)),
+                       dim3(kD18MergeThreads), 0, st, A, hd, doc_ptr);
+  }
   return check_launch();
+}
+
+extern "C" int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_docs, const float* qd,
+                             const float* qo, const void* k_docs, const void* v_docs, long long s_dh,
+                             long long s_dn, const int* doc_ptr, const float* k_own, const float* v_own,
+                             long long s_oh, long long s_on, int P, float scale, int skip, float beta,
+                             int top_k, int force, const float* wfix, int nsplit, float* out, float* w,
+                             float* r, float* rmax, void* workspace, size_t workspace_bytes, void* stream) {
+  const long long row = (long long)hq * hd;
+  return xenc_d18_read_strided(dtype, T, hq, hkv, hd, n_docs, qd, T * row, row, hd, qo, row, hd, k_docs, v_docs, s_dh,
+                               s_dn, doc_ptr, k_own, v_own, s_oh, s_on, P, scale, skip, beta, top_k, force, wfix,
+                               nsplit, out, w, r, rmax, nullptr, workspace, workspace_bytes, stream);
 }

@@ -57,25 +57,6 @@ __device__ __forceinline__ f32x16 mfma32(const half8_t& a, const half8_t& b, con
 // Instruction classes of __builtin_amdgcn_sched_group_barrier.
 constexpr int kSchedMfma = 0x008, kSchedVmemRead = 0x020, kSchedDsRead = 0x100;
 
-// One 16-byte chunk per lane from global memory straight into LDS (gfx950
-// global_load_lds_dwordx4): lane i of the wave writes lds_wave_base + 16 i.  lds_wave_base must
-// be wave-uniform.  Issued as inline assembly so that the compiler does not treat the LDS
-// write as pending at every barrier and LDS read (it would wait for every outstanding global
-// load there); the caller waits for these loads itself (wait_vmem) before publishing the LDS.
-__device__ __forceinline__ void stage_to_lds(_Float16* lds_wave_base, const _Float16* src) {
-  const unsigned lds = __builtin_amdgcn_readfirstlane(
-      (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)lds_wave_base);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
-}
-
-// Wait until at most N vector-memory operations of this wave are outstanding (they complete in
-// issue order for the counter).
-template <int N>
-__device__ __forceinline__ void wait_vmem() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 constexpr int kChunkGroup = 4;  // scores tiles: chunks per group, all row tiles of a group adjacent
 
 // Library g of tile b: tile_ptr[g] <= b < tile_ptr[g+1] (binary search; G is small).

@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass, field
+from functools import lru_cache
 
 import torch
 
@@ -1192,6 +1193,38 @@ def d18_nsplit(T: int, hkv: int, lengths, own: int) -> int:
     return max(1, min(32, want, max(max(lengths), own) // 128))
 
 
+_D18_TILE_ROWS = 16     # rows from which xenc_d18_read takes its tile kernel (csrc/d18.hip)
+
+
+@lru_cache(maxsize=256)
+def _d18_splits(T: int, hkv: int, G: int, hd: int, esize: int, n_docs: int, longest: int, own: int) -> int:
+    """Key splits of one call.  Few rows: d18_nsplit.  The tile kernel (a workgroup per 64 columns,
+    T * G per kv head; two fit a CU): the S with the least rounds of 512 workgroups x keys per split
+    (0.105 us a key at hd 256, 2.7 times that for fp32 keys) plus the partials' write and read (4
+    TB/s), keeping 128 to 2048 keys per split.  Measured at 130 rows x 16 heads, 4 documents of
+    1500 rows, bf16, hd 256: 119 / 88 / 71 / 80 / 79 us at 1 / 2 / 3 / 4 / 6 splits."""
+    if T < _D18_TILE_ROWS:
+        return d18_nsplit(T, hkv, [longest] * n_docs, own)
+    units = -(-T * G // 64) * hkv * n_docs
+    key = 0.105 * hd / 256 * (2.7 if esize == 4 else 1.0)
+    part = T * hkv * G * (n_docs + 1) * hd * 8 / 4e6
+
+    def cost(S):
+        return -(-units * S // 512) * (longest / S) * key + part * S
+
+    span = max(longest, own)
+    return min(range(max(1, -(-span // 2048)), max(1, min(32, span // 128)) + 1), key=cost)
+
+
+def _d18_rows(q: torch.Tensor) -> torch.Tensor:
+    """q [..., hd] in fp32, as the caller laid it out when every 16 bytes of a row can be loaded at
+    once (contiguous hd, strides and base multiples of 16 bytes), else a contiguous copy."""
+    q = q.detach().float()
+    if q.stride(-1) != 1 or any(s % 4 for s in q.stride()[:-1]) or q.data_ptr() % 16:
+        q = q.clone(memory_format=torch.contiguous_format)   # (contiguous() keeps a misaligned base)
+    return q
+
+
 def d18_read(qd: torch.Tensor, qo: torch.Tensor, ops, Kown: torch.Tensor, Vown: torch.Tensor, scale: float,
              skip: int = 0, beta: float = 1.0, top_k: int = 0, force: int | None = None,
              wfix: torch.Tensor | None = None, nsplit: int | None = None) -> dict:
@@ -1216,8 +1249,7 @@ def d18_read(qd: torch.Tensor, qo: torch.Tensor, ops, Kown: torch.Tensor, Vown: 
     dev = qd.device
     P = Kown.shape[1] - T
     G = Hq // Hkv
-    qd_ = qd.detach().float().transpose(1, 2).contiguous()          # [D, T, Hq, hd]
-    qo_ = qo.detach().float().transpose(0, 1).contiguous()          # [T, Hq, hd]
+    qd_, qo_ = _d18_rows(qd), _d18_rows(qo)
     ko, vo = Kown.detach().float().contiguous(), Vown.detach().float().contiguous()
     out = torch.empty(T, Hq, hd, dtype=torch.float32, device=dev)
     w = torch.empty(Hkv, G, T, D, dtype=torch.float32, device=dev)
@@ -1228,15 +1260,17 @@ def d18_read(qd: torch.Tensor, qo: torch.Tensor, ops, Kown: torch.Tensor, Vown: 
         wf = wfix.detach().to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
         if wf.numel() != D:
             raise ValueError("d18: wfix has one weight per document")
-    S = d18_nsplit(T, Hkv, P_ops.lengths, P + T) if nsplit is None else int(nsplit)
+    n = torch.empty(D, dtype=torch.float32, device=dev)
+    S = (_d18_splits(T, Hkv, G, hd, P_ops.K.element_size(), D, max(P_ops.lengths), P + T) if nsplit is None
+         else int(nsplit))
     nbytes = lib().xenc_d18_workspace_bytes(T, Hq, D, hd, S)
     ws = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=dev)
-    check(lib().xenc_d18_read(_D18_DTYPES[P_ops.K.dtype], T, Hq, Hkv, hd, D, ptr(qd_), ptr(qo_),
-                              ptr(P_ops.K), ptr(P_ops.V), P_ops.K.stride(0), P_ops.K.stride(1), ptr(P_ops.doc_ptr),
-                              ptr(ko), ptr(vo), ko.stride(0), ko.stride(1), P, float(scale), int(skip), float(beta),
-                              int(top_k), -1 if force is None else int(force), ptr(wf), S, ptr(out), ptr(w), ptr(r),
-                              ptr(rmax), ptr(ws), ws.numel(), stream_handle(dev)), "xenc_d18_read")
-    n = torch.tensor([float(m - skip) if m > skip else float(m) for m in P_ops.lengths], device=dev)
+    check(lib().xenc_d18_read_strided(
+        _D18_DTYPES[P_ops.K.dtype], T, Hq, Hkv, hd, D, ptr(qd_), qd_.stride(0), qd_.stride(2), qd_.stride(1), ptr(qo_),
+        qo_.stride(1), qo_.stride(0), ptr(P_ops.K), ptr(P_ops.V), P_ops.K.stride(0), P_ops.K.stride(1),
+        ptr(P_ops.doc_ptr), ptr(ko), ptr(vo), ko.stride(0), ko.stride(1), P, float(scale), int(skip), float(beta),
+        int(top_k), -1 if force is None else int(force), ptr(wf), S, ptr(out), ptr(w), ptr(r), ptr(rmax), ptr(n),
+        ptr(ws), ws.numel(), stream_handle(dev)), "xenc_d18_read_strided")
     return {"o": out.reshape(T, Hq * hd), "w": w, "r": r, "rmax": rmax, "n": n}
 
 
