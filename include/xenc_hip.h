@@ -425,6 +425,46 @@ int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_docs, const f
                   long long s_oh, long long s_on, int P, float scale, int skip, float beta,
                   int top_k, int force, const float* wfix, int nsplit, float* out, float* w,
                   float* r, float* rmax, void* workspace, size_t workspace_bytes, void* stream);
+/*
+ * ---- The read of many rows by entries (the pairs (row, chunk) that routing kept; csrc/entries.hip)
+ * Rows of library g are row_ptr[g] .. row_ptr[g+1]-1 (as in the prefill calls above).  Entry row * kk + j is
+ * rank j of the row: chunk idx[row, j] of its library (idx < 0: none).  M rows, n_chunks chunks in
+ * all, max_rows the most rows of one library.
+ * xenc_entries_list: list [n_chunks][max_rows], count [n_chunks]: each chunk's entries in row order.
+ * The calls below take those, or list = count = NULL: every row of a chunk's library, kk = the most
+ * chunks of a library and rank j = chunk j.  tile_rows (32, or 64 for pages of more than 128
+ * slots): entries per workgroup.
+ * xenc_entries_scores: modes, operands and results per entry as xenc_prefill_scores' per (row, chunk),
+ *   p and ds row-major [M * kk][slots] fp16, gamma [M * kk] (backward modes only).
+ * xenc_entries_readout: out[e] = scale * sum_n a[e, n] K[c, n], scale = w[row, c] when w != NULL;
+ *   by_row (kk = 1): into row e / kk of out.
+ * blocks = 1: a workgroup takes a whole chunk.  blocks = ceil(slots / 128) (forward modes, tile_rows
+ *   32): 128 slots each; mode 0 then writes 2^(s - m) with m the block's max rounded up, and stats
+ *   [M * kk][blocks] (m, sum), which the readout of that p takes (stats NULL: p as it stands).
+ * xenc_entries_merge: out[row] = sum_j part[row * kk + j] over the row's entries in rank order; S !=
+ *   NULL (backward): plus sum_j dl_j S[c_j], dl_j = route_temp w_j (dw_j - sum_i w_i dw_i), dw =
+ *   gamma (+ dw_ext [M, lde] when given).
+ * Limits as the prefill calls' (d and slots multiples of 64, slots <= 512).
+ * (xenc/injector.py:236-265 and its autograd)
+ */
+int xenc_entries_list(const int* idx, int M, int kk, const int* row_ptr, const int* chunk_ptr, int G,
+                      int n_chunks, int max_rows, int* list, int* count, void* stream);
+int xenc_entries_scores(int mode, const void* x, int M, int d, int kk, const int* row_ptr,
+                        const int* chunk_ptr, int G, int n_chunks, int max_rows, const int* list,
+                        const int* count, int tile_rows, const void* pages_a, int slots_per_page,
+                        long long page_stride, const int* chunk_page, const int* chunk_nvalid,
+                        float temp, const float* w, long long ldw, void* p, void* ds, float* gamma,
+                        int blocks, float* stats, void* stream);
+int xenc_entries_readout(const void* a, int M, int d, int kk, const int* row_ptr, const int* chunk_ptr,
+                         int G, int n_chunks, int max_rows, const int* list, const int* count,
+                         int tile_rows, const void* pages_b, int slots_per_page, long long page_stride,
+                         const int* chunk_page, const float* w, long long ldw, int by_row, int blocks,
+                         const float* stats, float* out, long long ldo, void* stream);
+int xenc_entries_merge(const float* part, int M, int d, int kk, const int* idx, const int* row_ptr,
+                       const int* chunk_ptr, int G, const float* w, long long ldw, const float* gamma,
+                       const float* dw_ext, long long lde, const float* S, float route_temp, float* out,
+                       long long ldo, void* stream);
+
 /* The same read of queries in any layout with hd contiguous (element strides, multiples of 4: qd by
  * document, row and head, qo by row and head), also writing n [D] fp32 (may be NULL): the keys of
  * document d that entered r_d, N_d - skip (N_d when N_d <= skip). */

@@ -139,6 +139,26 @@ SIGNATURES = {
         c_float, c_int, c_float, c_int, c_int, c_void_p, c_int,  # scale, skip, beta, top_k, force, wfix, nsplit
         c_void_p, c_void_p, c_void_p, c_void_p,      # out, w, r, rmax
         c_void_p, c_size_t, c_void_p]),              # workspace, workspace_bytes, stream
+    "xenc_entries_list": (c_int, [
+        c_void_p, c_int, c_int, c_void_p, c_void_p,  # idx, M, kk, row_ptr, chunk_ptr
+        c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),  # G, n_chunks, max_rows, list, count, stream
+    "xenc_entries_scores": (c_int, [
+        c_int, c_void_p, c_int, c_int, c_int,        # mode, x, M, d, kk
+        c_void_p, c_void_p, c_int, c_int, c_int,     # row_ptr, chunk_ptr, G, n_chunks, max_rows
+        c_void_p, c_void_p, c_int, c_void_p, c_int,  # list, count, tile_rows, pages_a, slots
+        c_longlong, c_void_p, c_void_p, c_float,     # page_stride, chunk_page, chunk_nvalid, temp
+        c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,  # w, ldw, p, ds, gamma
+        c_int, c_void_p, c_void_p]),                 # blocks, stats, stream
+    "xenc_entries_readout": (c_int, [
+        c_void_p, c_int, c_int, c_int, c_void_p, c_void_p,  # a, M, d, kk, row_ptr, chunk_ptr
+        c_int, c_int, c_int, c_void_p, c_void_p, c_int,     # G, n_chunks, max_rows, list, count, tile_rows
+        c_void_p, c_int, c_longlong, c_void_p,       # pages_b, slots, page_stride, chunk_page
+        c_void_p, c_longlong, c_int, c_int, c_void_p,  # w, ldw, by_row, blocks, stats
+        c_void_p, c_longlong, c_void_p]),            # out, ldo, stream
+    "xenc_entries_merge": (c_int, [
+        c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int,  # part, M, d, kk, idx, row_ptr, chunk_ptr, G
+        c_void_p, c_longlong, c_void_p, c_void_p, c_longlong,  # w, ldw, gamma, dw_ext, lde
+        c_void_p, c_float, c_void_p, c_longlong, c_void_p]),   # S, route_temp, out, ldo, stream
     "xenc_d18_read_strided": (c_int, [
         c_int, c_int, c_int, c_int, c_int, c_int,    # dtype, T, hq, hkv, hd, n_docs
         c_void_p, c_longlong, c_longlong, c_longlong,  # qd, strides (document, row, head)

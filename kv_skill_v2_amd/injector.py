@@ -98,6 +98,12 @@ def write_delta(itf, hn: torch.Tensor, r: torch.Tensor, li: int, gain_scale: flo
     return out.view(*r.shape[:-1], B.weight.shape[0])
 
 
+def _by_entries(rows: int) -> bool:
+    """Prompts read their routed pairs; a decode step's batch (the rows of the fused write-back) keeps
+    the 128-row tiles, so that a generated sequence's residual stream keeps its bits."""
+    return rows > _FUSED_WRITE_ROWS
+
+
 # ----------------------------------------------------------------------------- hooks
 class _AddUpdate:
     """Forward hook of one injection layer: the layer's output hidden state plus the branch's
@@ -214,8 +220,9 @@ class XEncInjector(SkillInjector):
     def _branch(self, h: torch.Tensor, li: int) -> torch.Tensor:
         hn, q = self._query(h)
         lead, d = q.shape[:-1], q.shape[-1]
-        r, _ = ops.branch_read(q.reshape(-1, d), self._skill_pool(li, hn.device), 0, self.read_temp, 1.0,
-                               self.read_softmax)
+        rows = q.reshape(-1, d)
+        r, _ = ops.branch_read(rows, self._skill_pool(li, hn.device), 0, self.read_temp, 1.0, self.read_softmax,
+                               _by_entries(rows.shape[0]))
         r, gcal = self._calibrated(r.view(*lead, -1), li)
         return write_delta(self.itf, hn, r, li, self.gain_scale, gcal)
 
@@ -299,11 +306,12 @@ class LibraryInjector(XEncInjector):
         rows = q.reshape(-1, d)
         if keep is None or (torch.is_grad_enabled() and rows.requires_grad):
             # (with autograd every row is read: the selector's weight zeroes the left-out ones)
-            r, w = ops.branch_read(rows, pool, self.top_k, self.read_temp, self.route_temp, self.read_softmax)
+            r, w = ops.branch_read(rows, pool, self.top_k, self.read_temp, self.route_temp, self.read_softmax,
+                                   _by_entries(rows.shape[0]))
             return r.view(*lead, -1), w.view(*lead, -1)
         w, idx, w_sel = ops.route_rows(rows, pool, self.top_k, self.route_temp)
         idx = torch.where(keep.reshape(-1, 1), idx, torch.full_like(idx, -1))
-        r = ops.read_rows(rows, w, idx, w_sel, pool, self.read_temp, self.read_softmax)
+        r = ops.read_rows(rows, w, idx, w_sel, pool, self.read_temp, self.read_softmax, _by_entries(rows.shape[0]))
         return r.view(*lead, -1), w.view(*lead, -1)
 
     def _slot_attention(self, q_rows: torch.Tensor, w_rows: torch.Tensor, li: int) -> torch.Tensor:

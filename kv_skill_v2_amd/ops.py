@@ -920,6 +920,16 @@ def library_read(q: torch.Tensor, lib_: PagedLibrary, plan: RowPlan, top_k: int 
             raise ValueError(f"q must have {plan.M} rows")
         fk, fv, fvs, fkr, chunk_ptr, chunk_page, chunk_nvalid, row_ptr, score_tiles, readout_tiles, n_score, \
             n_readout, slots = _prefill_operands(lib_, plan)
+        kk = lib_.kept(int(top_k))
+        # The routed (row, chunk) pairs only; reading every chunk without a gradient stays equal, bit for
+        # bit, to route_topk_rows and prefill_forward.
+        grad = torch.is_grad_enabled() and q.requires_grad
+        tile = _entry_tile(plan.rows, lib_, kk) if grad or kk < lib_.cmax else 0
+        if tile:
+            return torch.ops.xenc.library_read_entries(
+                q, lib_.S, chunk_ptr, row_ptr, plan.logit_tiles, plan.route_tiles, plan.n_logit, plan.n_route,
+                int(top_k), float(route_temp), lib_.cmax, kk, fk, fv, fvs, fkr, chunk_page, chunk_nvalid,
+                max(plan.rows), tile, slots, float(read_temp), bool(read_softmax))[:2]
         r, w, _, _, _ = torch.ops.xenc.library_read_routed(
             q, lib_.S, chunk_ptr, row_ptr, plan.logit_tiles, plan.route_tiles, plan.n_logit, plan.n_route,
             int(top_k), float(route_temp), lib_.cmax, lib_.kept(int(top_k)), fk, fv, fvs, fkr, chunk_page,
@@ -1077,6 +1087,53 @@ def prefill_ok(lib_: PagedLibrary) -> bool:
     return lib_.d % 64 == 0 and lib_.slots_per_page % 64 == 0 and lib_.slots_per_page <= 512
 
 
+def _entry_tile(rows: list[int], lib_: PagedLibrary, kk: int) -> int:
+    """0: read every row against every chunk in 128-row tiles (csrc/prefill.hip); 32 or 64: read the
+    kept (row, chunk) pairs grouped by chunk, that many per workgroup (csrc/entries.hip)."""
+    pairs = list(zip(rows, lib_.n_chunks))
+    return _entry_tile_of(sum(-(-m // 128) * c for m, c in pairs), sum(-(-m // 128) for m in rows),
+                          sum(m * min(c, kk) for m, c in pairs), sum(lib_.n_chunks), lib_.cmax, kk,
+                          lib_.slots_per_page, lib_.d)
+
+
+@lru_cache(maxsize=1024)
+def _entry_tile_of(tiles: int, row_tiles: int, entries: int, n_chunks: int, cmax: int, kk: int, N: int, d: int) -> int:
+    """The cheaper by this model, in us, fitted to measured forward kernels (the backward repeats the
+    same two products, so the order holds for it).  Dense: a scores round of 256 workgroups 48 (a
+    full one 65), a readout k step 1.05, both at d = 2048.  Entries: a scores round 31 (32 rows) or 42
+    (64), a readout workgroup's 22 or 42 ns of the GPU, the partials' read at 6 TB/s, lists and launches.
+    Measured per call, dense against entries: 333 rows, top-4 of 16 chunks of 512 x 2048 208 / 57
+    us; 1000 rows, top-8 and all of 16: 218 / 126 and 218 / 177; 2048 rows, top-8 of 64: 858 / 308;
+    2048 rows, top-4 of 8: 176 / 140; a training step of 4 x 2048 rows, top-4 of 32: 2.22 / 1.04 ms."""
+    D = d / 2048
+    dense = max(48, 65 * tiles / 256) * D + 1.05 * cmax * (N / 64) * max(1, row_tiles * -(-d // 256) / 256)
+    best, tile = dense, 0
+    for rt, scores, out in ((32, 31, 0.022), (64, 42, 0.042)):
+        if rt == 64 and N <= 128:
+            continue
+        t = entries / rt + (n_chunks / 2 if kk < cmax else 0)   # (a chunk's last tile is half full on average)
+        cost = scores * D * max(N, 128) / 512 * max(1, math.ceil(t / 256)) + 8 + t * -(-d // 256) * out * N / 512 + 6
+        if kk > 1:
+            cost += entries * d * 4 / 6e6 + 3
+        if cost < best:
+            best, tile = cost, rt
+    return tile
+
+
+def _read_entries(q: torch.Tensor, w: torch.Tensor, idx: torch.Tensor | None, lib_: PagedLibrary, tile: int,
+                  read_temp: float, read_softmax: bool) -> torch.Tensor:
+    """r [M, d] of M rows of one library by entries: those of idx [M, kk], or (None) every chunk."""
+    plan = lib_.plan([q.shape[0]])
+    # Tiles that leave CUs idle are split by 128 slots too (a tile is bound by one CU's loads).
+    kk = lib_.cmax if idx is None else idx.shape[1]
+    split = tile == 32 and lib_.slots_per_page > 128 and q.shape[0] * kk // 32 + lib_.cmax // 2 < 128
+    return torch.ops.xenc.read_entries(
+        _query(q, lib_.d), w.to(torch.float32).contiguous(), idx, lib_.fragment_pages(0),
+        lib_.fragment_pages(1, values=True), lib_.chunk_ptr, plan.row_ptr, lib_.chunk_page, lib_.chunk_nvalid,
+        q.shape[0], tile, -(-lib_.slots_per_page // 128) if split else 1, lib_.slots_per_page, float(read_temp),
+        bool(read_softmax))
+
+
 def _pad_rows(q: torch.Tensor, lib_: PagedLibrary) -> torch.Tensor:
     _require_device(q, "q")
     if q.dim() != 2 or q.shape[1] != lib_.d_valid:
@@ -1102,7 +1159,8 @@ def route_rows(q: torch.Tensor, lib_: PagedLibrary, top_k: int = 0, route_temp: 
 
 
 def read_rows(q: torch.Tensor, w: torch.Tensor, idx: torch.Tensor, w_sel: torch.Tensor,
-              lib_: PagedLibrary, read_temp: float = 12.0, read_softmax: bool = True) -> torch.Tensor:
+              lib_: PagedLibrary, read_temp: float = 12.0, read_softmax: bool = True,
+              by_entries: bool = True) -> torch.Tensor:
     """r [M, d_valid]: the read of M query rows over ONE library given their routing (the read of
     LibraryInjector._branch, xenc/injector.py:239-265).
 
@@ -1117,7 +1175,15 @@ def read_rows(q: torch.Tensor, w: torch.Tensor, idx: torch.Tensor, w_sel: torch.
     mfma = grad or lib_.values is not None or M > DECODE_MAX_ROWS
     if mfma and not prefill_ok(lib_) and not (grad or lib_.values is not None):
         mfma = False        # a forward read of larger pages: the split-K decode path takes any size
-    if mfma and prefill_ok(lib_):
+    # (launches of few 128-row tiles: every (row, chunk) pair as an entry, weighted by w)
+    tile = 0
+    if by_entries and mfma and not grad and prefill_ok(lib_):
+        tile = _entry_tile([M], lib_, lib_.cmax)
+    if tile:
+        if w.shape != (M, lib_.cmax):
+            raise ValueError(f"w must have shape ({M}, {lib_.cmax})")
+        r = _read_entries(qp, w, None, lib_, tile, read_temp, read_softmax)
+    elif mfma and prefill_ok(lib_):
         r, _ = prefill_forward(qp, w, lib_, lib_.plan([M]), float(read_temp), bool(read_softmax))
     elif mfma:
         if not _mfma_pages_ok(lib_):
@@ -1129,19 +1195,25 @@ def read_rows(q: torch.Tensor, w: torch.Tensor, idx: torch.Tensor, w_sel: torch.
 
 
 def branch_read(q: torch.Tensor, lib_: PagedLibrary, top_k: int = 0, read_temp: float = 12.0,
-                route_temp: float = 10.0, read_softmax: bool = True):
-    """(r [M, d_valid], w [M, C]): route_rows + read_rows.  Under autograd with at least
-    ROUTE_ROWS_MIN rows (and a pool the MFMA read takes), library_read instead: routing and read as
-    one operator."""
+                route_temp: float = 10.0, read_softmax: bool = True, by_entries: bool = True):
+    """(r [M, d_valid], w [M, C]): route_rows + read_rows, many rows by their routed pairs where that is
+    the cheaper read (by_entries).  Under autograd with at least ROUTE_ROWS_MIN rows (and a pool the
+    MFMA read takes), library_read instead: routing and read as one operator."""
     _single(lib_)
     M = q.shape[0]
-    if (torch.is_grad_enabled() and q.requires_grad and prefill_ok(lib_) and M >= ROUTE_ROWS_MIN
-            and lib_.cmax <= 1024):
+    grad = torch.is_grad_enabled() and q.requires_grad
+    if grad and prefill_ok(lib_) and M >= ROUTE_ROWS_MIN and lib_.cmax <= 1024:
         r, w = library_read(_pad_rows(q, lib_), lib_, lib_.plan([M]), int(top_k), float(read_temp),
                             float(route_temp), bool(read_softmax))
         return (r[:, :lib_.d_valid] if lib_.d != lib_.d_valid else r), w
+    tile = 0
+    if by_entries and not grad and prefill_ok(lib_) and (M > DECODE_MAX_ROWS or lib_.values is not None):
+        tile = _entry_tile([M], lib_, lib_.kept(int(top_k)))
     w, idx, wsel = route_rows(q, lib_, top_k, route_temp)
-    return read_rows(q, w, idx, wsel, lib_, read_temp, read_softmax), w
+    if tile:   # the pairs the routing kept
+        r = _read_entries(_pad_rows(q, lib_), w, idx, lib_, tile, read_temp, read_softmax)
+        return (r[:, :lib_.d_valid] if lib_.d != lib_.d_valid else r), w
+    return read_rows(q, w, idx, wsel, lib_, read_temp, read_softmax, by_entries), w
 
 
 # ----------------------------------------------------------------------------- D18 multi-document read

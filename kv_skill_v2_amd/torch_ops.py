@@ -23,6 +23,9 @@ dispatcher, FakeTensor tracing and torch.compile see ordinary operators:
     xenc::library_prefill_bwd_routed  dq through the read and the routing in one pass over dq
     xenc::library_read_routed    route_rows + library_prefill_fwd as one autograd node (its
                                  backward is library_prefill_bwd_routed)
+    xenc::library_read_entries   the same over the routed (row, chunk) pairs only, grouped by chunk
+                                 (its backward is library_read_entries_bwd); xenc::read_entries is
+                                 its read of rows already routed, without a gradient
     xenc::paged_decode_joint     DecodeReader's joint read (xenc/d23_read_kernels.py:145-160) into
                                  a caller-owned output; writes its workspace
 
@@ -138,6 +141,7 @@ def _route_rows_setup(ctx, inputs, output):
     ctx.save_for_backward(w, S, chunk_ptr, row_ptr, route_tiles)
     ctx.n_route, ctx.route_temp, ctx.d = n_route, route_temp, q.shape[1]
     ctx.mark_non_differentiable(output[1], output[2], output[3])
+    ctx.set_materialize_grads(False)   # (else every backward fills zeros for p, idx and w_sel)
 
 
 def _route_rows_backward(ctx, dw, _didx, _dwsel, _dqh):
@@ -298,6 +302,7 @@ def _prefill_setup(ctx, inputs, output):
                           readout_tiles)
     ctx.sizes = (n_score, n_readout, slots, read_temp, softmax)
     ctx.mark_non_differentiable(output[1])
+    ctx.set_materialize_grads(False)   # (else every backward fills zeros for p, idx and w_sel)
 
 
 def _prefill_backward(ctx, dr, _dp):
@@ -351,6 +356,7 @@ def _routed_setup(ctx, inputs, output):
     ctx.route = (n_route, route_temp)
     ctx.d = q.shape[1]
     ctx.mark_non_differentiable(output[2], output[3], output[4])
+    ctx.set_materialize_grads(False)   # (else every backward fills zeros for p, idx and w_sel)
 
 
 def _routed_backward(ctx, dr, dw, _didx, _dwsel, _dp):
@@ -370,6 +376,57 @@ def _routed_backward(ctx, dr, dw, _didx, _dwsel, _dp):
 
 
 library_read_routed.register_autograd(_routed_backward, setup_context=_routed_setup)
+
+
+# ----------------------------------------------------------------------------- the read by entries
+# (csrc/entries.hip; defined and implemented in csrc/torch_ops.cpp)
+@torch.library.register_fake("xenc::read_entries")
+def _(q, w, idx, frag_k_scores, frag_v_readout, chunk_ptr, row_ptr, chunk_page, chunk_nvalid, max_rows, tile_rows,
+      blocks, slots, read_temp, softmax):
+    return q.new_empty(q.shape)
+
+
+@torch.library.register_fake("xenc::library_read_entries")
+def _(q, S, chunk_ptr, row_ptr, logit_tiles, route_tiles, n_logit, n_route, top_k, route_temp, cmax, kk,
+      frag_k_scores, frag_v_readout, frag_v_scores, frag_k_readout, chunk_page, chunk_nvalid, max_rows, tile_rows,
+      slots, read_temp, softmax):
+    M, C = q.shape[0], chunk_page.shape[0]
+    return (q.new_empty(q.shape), q.new_empty(M, cmax), q.new_empty(M, kk, dtype=torch.int32), q.new_empty(M, kk),
+            q.new_empty(M * kk, slots, dtype=torch.float16), q.new_empty(C, max_rows, dtype=torch.int32),
+            q.new_empty(C, dtype=torch.int32))
+
+
+@torch.library.register_fake("xenc::library_read_entries_bwd")
+def _(g, w, idx, p, dw_ext, S, list, count, frag_v_scores, frag_k_readout, chunk_ptr, chunk_page, chunk_nvalid, row_ptr,
+      max_rows, tile_rows, slots, read_temp, softmax, route_temp):
+    return g.new_empty(g.shape)
+
+
+def _entries_setup(ctx, inputs, output):
+    (q, S, chunk_ptr, row_ptr, _lt, route_tiles, _nl, n_route, _tk, route_temp, _cmax, _kk, _fks, _fvr, fvs, fkr,
+     chunk_page, chunk_nvalid, max_rows, tile_rows, slots, read_temp, softmax) = inputs
+    _, w, idx, _, p, lst, count = output
+    ctx.save_for_backward(w, idx, p, lst, count, fvs, fkr, chunk_ptr, chunk_page, chunk_nvalid, row_ptr, S, route_tiles)
+    ctx.sizes = (max_rows, tile_rows, slots, read_temp, softmax)
+    ctx.route = (n_route, route_temp)
+    ctx.d = q.shape[1]
+    ctx.mark_non_differentiable(*output[2:])
+    ctx.set_materialize_grads(False)   # (else every backward fills zeros for p, idx and w_sel)
+
+
+def _entries_backward(ctx, dr, dw, *_):
+    w, idx, p, lst, count, fvs, fkr, chunk_ptr, chunk_page, chunk_nvalid, row_ptr, S, route_tiles = ctx.saved_tensors
+    dw = None if dw is None else dw.contiguous()
+    if dr is None:  # only w reaches the loss: the routing term alone
+        dq = torch.zeros(w.shape[0], ctx.d, dtype=torch.float32, device=w.device)
+        torch.ops.xenc.route_backward_(dq, w, torch.zeros_like(w), dw, S, chunk_ptr, row_ptr, route_tiles, *ctx.route)
+    else:
+        dq = torch.ops.xenc.library_read_entries_bwd(dr.contiguous(), w, idx, p, dw, S, lst, count, fvs, fkr, chunk_ptr,
+                                                     chunk_page, chunk_nvalid, row_ptr, *ctx.sizes, ctx.route[1])
+    return (dq,) + (None,) * 22
+
+
+torch.library.register_autograd("xenc::library_read_entries", _entries_backward, setup_context=_entries_setup)
 
 
 # ----------------------------------------------------------------------------- op B
