@@ -368,6 +368,15 @@ int xenc_topk_rows(const float* scores, long long ld_s, int B, int S, int k, int
 int xenc_gather_pages(const void* pages, int slots_per_page, long long page_stride, int d,
                       const int* chunk_page, int n_chunks, int n_flat, const int* idx,
                       long long ld_idx, int G, int k, int kpad, void* out, void* stream);
+/* The same copy, and with S_out / meta (both or neither) what makes the G sets one library of one chunk
+ * each: S_out [G][d] = 0, meta int32 [3 G + 1] = page table (g) | valid slots (k) | chunk offsets. */
+int xenc_gather_library(const void* pages, int slots_per_page, long long page_stride, int d,
+                        const int* chunk_page, int n_chunks, int n_flat, const int* idx, long long ld_idx,
+                        int G, int k, int kpad, void* out, float* S_out, int* meta, void* stream);
+/* n <= 256 integers from host memory (read before the call returns) into device memory `out`, passed
+ * as kernel arguments: capturable, no copy to wait for. */
+int xenc_store_ints(const int* values, int n, int* out, void* stream);
+
 
 /*
  * ---- Op B serving step (per-request decode state on the device)

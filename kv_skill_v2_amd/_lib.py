@@ -139,6 +139,11 @@ SIGNATURES = {
         c_float, c_int, c_float, c_int, c_int, c_void_p, c_int,  # scale, skip, beta, top_k, force, wfix, nsplit
         c_void_p, c_void_p, c_void_p, c_void_p,      # out, w, r, rmax
         c_void_p, c_size_t, c_void_p]),              # workspace, workspace_bytes, stream
+    "xenc_gather_library": (c_int, [
+        c_void_p, c_int, c_longlong, c_int,          # pages, slots_per_page, page_stride, d
+        c_void_p, c_int, c_int, c_void_p, c_longlong,  # chunk_page, n_chunks, n_flat, idx, ld_idx
+        c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p]),  # G, k, kpad, out, S_out, meta, stream
+    "xenc_store_ints": (c_int, [c_void_p, c_int, c_void_p, c_void_p]),  # values, n, out, stream
     "xenc_entries_list": (c_int, [
         c_void_p, c_int, c_int, c_void_p, c_void_p,  # idx, M, kk, row_ptr, chunk_ptr
         c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),  # G, n_chunks, max_rows, list, count, stream

@@ -151,6 +151,28 @@ __global__ __launch_bounds__(kPoolWaves * kWave) void build_pages_kernel(
 
 using namespace xenc;
 
+// A few integers from the host into device memory as kernel arguments: no staging copy to wait for.
+namespace xenc {
+namespace {
+struct Ints {
+  int v[256];
+};
+__global__ __launch_bounds__(256) void store_ints_kernel(const Ints a, int n, int* __restrict__ out) {
+  if ((int)threadIdx.x < n) out[threadIdx.x] = a.v[threadIdx.x];
+}
+}  // namespace
+}  // namespace xenc
+
+extern "C" int xenc_store_ints(const int* values, int n, int* out, void* stream) {
+  if (n < 0 || n > 256) return XENC_EINVAL;
+  if (n == 0) return XENC_OK;
+  if (!values || !out) return XENC_ENULL;
+  Ints a = {};
+  std::copy(values, values + n, a.v);
+  hipLaunchKernelGGL(store_ints_kernel, dim3(1), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a, n, out);
+  return check_launch();
+}
+
 extern "C" int xenc_build_pages(const void* rows, const long long* row_off, int C, int d,
                                 const float* mu, int slots_per_page, int d_pad, void* pages,
                                 long long page_stride, float* S, long long lds, int* nvalid,

@@ -10,6 +10,7 @@ Every function here requires ROCm device tensors and raises otherwise: there is 
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass, field
 from functools import lru_cache
@@ -114,6 +115,13 @@ class PagedLibrary:
             self.d_valid = d
 
     # ------------------------------------------------------------------ constructors
+    @classmethod
+    def _unchecked(cls, **fields) -> "PagedLibrary":
+        """A pool whose fields (all of the public ones) the caller has made consistent."""
+        p = object.__new__(cls)
+        p.__dict__.update(fields, _frag={}, _plans={}, _kept={})
+        return p
+
     @staticmethod
     def from_padded(K: torch.Tensor, mask: torch.Tensor, S: torch.Tensor, device=None, V=None,
                     pad_to: int = 1) -> "PagedLibrary":
@@ -660,7 +668,8 @@ def select_scores(q: torch.Tensor, keys: torch.Tensor, valid: torch.Tensor | Non
         _require_device(valid, "valid")
         if valid.numel() != S:
             raise ValueError(f"valid must have {S} entries")
-        vb = valid.reshape(-1).to(torch.uint8).contiguous()
+        vb = valid.reshape(-1).contiguous()
+        vb = vb.view(torch.uint8) if vb.dtype == torch.bool else vb.to(torch.uint8)
     out = torch.empty(B, S, dtype=torch.float32, device=q.device)
     check(lib().xenc_select_scores(ptr(q), B, n_q, n_kv, hd, ptr(keys), S, ptr(vb), int(pool == "mean"),
                                    ptr(out), out.stride(0), stream_handle(q.device)), "xenc_select_scores")
@@ -698,20 +707,20 @@ def gather_library(lib_: PagedLibrary, idx: torch.Tensor, n_flat: int, pad_to: i
     ii = idx.to(torch.int32).contiguous()
     dev = lib_.device
 
-    def gather(src):
+    def gather(src, S=None, meta=None):
         out = torch.empty(G, kpad, lib_.d, dtype=torch.float16, device=dev)
-        check(lib().xenc_gather_pages(ptr(src), lib_.slots_per_page, lib_.slots_per_page * lib_.d, lib_.d,
-                                      ptr(lib_.chunk_page), lib_.chunk_page.numel(), int(n_flat), ptr(ii), k,
-                                      G, k, kpad, ptr(out), stream_handle(dev)), "xenc_gather_pages")
+        check(lib().xenc_gather_library(ptr(src), lib_.slots_per_page, lib_.slots_per_page * lib_.d, lib_.d,
+                                        ptr(lib_.chunk_page), lib_.chunk_page.numel(), int(n_flat), ptr(ii), k, G, k,
+                                        kpad, ptr(out), ptr(S), ptr(meta), stream_handle(dev)), "xenc_gather_library")
         return out
 
-    pages = gather(lib_.pages)
+    S = torch.empty(G, lib_.d, dtype=torch.float32, device=dev)
+    meta = torch.empty(3 * G + 1, dtype=torch.int32, device=dev)
+    pages = gather(lib_.pages, S, meta)
     values = gather(lib_.values) if lib_.values is not None else None
-    return PagedLibrary(pages, torch.arange(G, dtype=torch.int32, device=dev),
-                        torch.full((G,), k, dtype=torch.int32, device=dev),
-                        torch.arange(G + 1, dtype=torch.int32, device=dev),
-                        torch.zeros(G, lib_.d, dtype=torch.float32, device=dev),
-                        n_chunks=[1] * G, nvalid=[k] * G, values=values, d_valid=lib_.d_valid)
+    # Valid by construction: no check that would read the device back.
+    return PagedLibrary._unchecked(pages=pages, chunk_page=meta[:G], chunk_nvalid=meta[G:2 * G], chunk_ptr=meta[2 * G:],
+                                   S=S, n_chunks=[1] * G, nvalid=[k] * G, values=values, d_valid=lib_.d_valid)
 
 
 def _prefix(counts) -> list[int]:
@@ -752,8 +761,19 @@ def row_plan(lib_: PagedLibrary, rows_per_library) -> RowPlan:
     ro = _prefix(-(-t // ROWS_READOUT) * d_tiles for t in rows)
     rb = _prefix(-(-t // ROWS_ROUTE_BWD) for t in rows)
     lg = _prefix(-(-t // ROUTE_TILE) * -(-c // ROUTE_TILE) for t, c in zip(rows, lib_.n_chunks))
-    return RowPlan(rows, _i32(_prefix(rows), dev), _i32(sc, dev), sc[-1], _i32(ro, dev), ro[-1],
-                   _i32(rb, dev), rb[-1], _i32(lg, dev), lg[-1])
+    # The five offset tables in one buffer (each from a 16-byte boundary), one launch or one copy.
+    tables, host = [_prefix(rows), sc, ro, rb, lg], []
+    for t in tables:
+        host += t + [0] * (-len(t) % 4)
+    if len(host) <= 256:
+        buf = torch.empty(len(host), dtype=torch.int32, device=dev)
+        check(lib().xenc_store_ints((ctypes.c_int * len(host))(*host), len(host), ptr(buf), stream_handle(buf.device)),
+              "xenc_store_ints")
+    else:
+        buf = _i32(host, dev)
+    step = len(host) // 5
+    row_ptr, sc_t, ro_t, rb_t, lg_t = (buf[i * step:i * step + len(rows) + 1] for i in range(5))
+    return RowPlan(rows, row_ptr, sc_t, sc[-1], ro_t, ro[-1], rb_t, rb[-1], lg_t, lg[-1])
 
 
 def cast_f16(x: torch.Tensor) -> torch.Tensor:
