@@ -435,6 +435,17 @@ int xenc_d18_read(int dtype, int T, int hq, int hkv, int hd, int n_docs, const f
                   int top_k, int force, const float* wfix, int nsplit, float* out, float* w,
                   float* r, float* rmax, void* workspace, size_t workspace_bytes, void* stream);
 /*
+ * ---- The row-wise work of a hooked layer (xenc/injector.py:54-58, 185-197; fp32, rows of d % 4 == 0
+ * columns, row strides multiples of 4, 16-byte aligned bases)
+ * xenc_hook_norm: hn [M][d] = h * rsqrt(mean(h^2) + eps);  xenc_hook_unit: q /= |q| + eps, in place;
+ * xenc_hook_add: out [M][d] = h + delta, ratio [M] = |delta| / (|h| + 1e-6).
+ */
+int xenc_hook_norm(const float* h, long long ldh, int M, int d, float eps, float* hn, void* stream);
+int xenc_hook_unit(float* q, long long ldq, int M, int d, float eps, void* stream);
+int xenc_hook_add(const float* h, long long ldh, const float* delta, long long ldd, int M, int d,
+                  float* out, float* ratio, void* stream);
+
+/*
  * ---- The read of many rows by entries (the pairs (row, chunk) that routing kept; csrc/entries.hip)
  * Rows of library g are row_ptr[g] .. row_ptr[g+1]-1 (as in the prefill calls above).  Entry row * kk + j is
  * rank j of the row: chunk idx[row, j] of its library (idx < 0: none).  M rows, n_chunks chunks in

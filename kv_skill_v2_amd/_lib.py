@@ -139,6 +139,13 @@ SIGNATURES = {
         c_float, c_int, c_float, c_int, c_int, c_void_p, c_int,  # scale, skip, beta, top_k, force, wfix, nsplit
         c_void_p, c_void_p, c_void_p, c_void_p,      # out, w, r, rmax
         c_void_p, c_size_t, c_void_p]),              # workspace, workspace_bytes, stream
+    "xenc_hook_norm": (c_int, [
+        c_void_p, c_longlong, c_int, c_int, c_float, c_void_p, c_void_p]),  # h, ldh, M, d, eps, hn, stream
+    "xenc_hook_unit": (c_int, [
+        c_void_p, c_longlong, c_int, c_int, c_float, c_void_p]),  # q, ldq, M, d, eps, stream
+    "xenc_hook_add": (c_int, [
+        c_void_p, c_longlong, c_void_p, c_longlong,  # h, ldh, delta, ldd
+        c_int, c_int, c_void_p, c_void_p, c_void_p]),  # M, d, out, ratio, stream
     "xenc_gather_library": (c_int, [
         c_void_p, c_int, c_longlong, c_int,          # pages, slots_per_page, page_stride, d
         c_void_p, c_int, c_int, c_void_p, c_longlong,  # chunk_page, n_chunks, n_flat, idx, ld_idx

@@ -11,6 +11,9 @@
 //   xenc::read_entries        the read of many rows by their routed (row, chunk) pairs, no gradient
 //   xenc::library_read_entries, library_read_entries_bwd   routing + that read, and its dQ (autograd
 //                             registered in torch_ops.py)
+//   xenc::hook_query, hook_write, hook_add   a hooked layer's query, update and residual add around
+//                             the read, for steps without a gradient
+//   xenc::hook_layer          a whole hooked layer of a decode step: the above and route_read
 //   xenc::paged_decode_joint  DecodeReader.__call__ (xenc/d23_read_kernels.py:145-160)
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
@@ -259,6 +262,73 @@ at::Tensor library_read_entries_bwd(const at::Tensor& g, const at::Tensor& w, co
                    route_temp);
 }
 
+// ---- a hooked layer around its read (xenc/injector.py:54-77, 185-197)
+// (hn, q) of rows h [M, d_m]: hn = rms_norm(h), q = A hn / (|A hn| + eps).
+std::tuple<at::Tensor, at::Tensor> hook_query(const at::Tensor& h, const at::Tensor& A,
+                                              const c10::optional<at::Tensor>& bias, double eps) {
+  const c10::DeviceGuard guard(h.device());
+  void* st = stream_of(h);
+  at::Tensor hn = at::empty({h.size(0), h.size(1)}, f32(h));
+  check(xenc_hook_norm(ptr<const float>(h), h.stride(0), (int)h.size(0), (int)h.size(1), (float)eps, ptr<float>(hn), st),
+        "xenc_hook_norm");
+  at::Tensor q = at::linear(hn, A, bias);
+  check(xenc_hook_unit(ptr<float>(q), q.stride(0), (int)q.size(0), (int)q.size(1), (float)eps, st), "xenc_hook_unit");
+  return {hn, q};
+}
+
+// delta [M, d_out] = scale * (W r + bias), scale = gain_scale exp(log_gain) sigmoid(hn . gate_w + gate_b).
+at::Tensor hook_write(const at::Tensor& hn, const at::Tensor& r, const at::Tensor& gate_w, const at::Tensor& gate_b,
+                      const at::Tensor& log_gain, double gain_scale, const at::Tensor& W,
+                      const c10::optional<at::Tensor>& bias) {
+  const c10::DeviceGuard guard(r.device());
+  void* st = stream_of(r);
+  const int M = (int)r.size(0), d = (int)r.size(1), d_out = (int)W.size(0);
+  at::Tensor scale = at::empty({M}, f32(r)), out = at::empty({M, d_out}, f32(r));
+  check(xenc_gate_scale(M, (int)hn.size(1), ptr<const float>(hn), hn.stride(0), nullptr, nullptr, 1,
+                        ptr<const float>(gate_w), ptr<const float>(gate_b), ptr<const float>(log_gain),
+                        (float)gain_scale, ptr<float>(scale), st),
+        "xenc_gate_scale");
+  check(xenc_write_back(ptr<const float>(r), r.stride(0), M, d, nullptr, 1, ptr<const float>(W),
+                        (long long)d_out * W.stride(0), W.stride(0), d_out, bias ? ptr<const float>(*bias) : nullptr, 0,
+                        ptr<const float>(scale), ptr<float>(out), out.stride(0), st),
+        "xenc_write_back");
+  return out;
+}
+
+// (h + delta, |delta| / (|h| + 1e-6) per row) of rows h, delta [M, d].
+std::tuple<at::Tensor, at::Tensor> hook_add(const at::Tensor& h, const at::Tensor& delta) {
+  const c10::DeviceGuard guard(h.device());
+  at::Tensor out = at::empty({h.size(0), h.size(1)}, f32(h)), ratio = at::empty({h.size(0)}, f32(h));
+  check(xenc_hook_add(ptr<const float>(h), h.stride(0), ptr<const float>(delta), delta.stride(0), (int)h.size(0),
+                      (int)h.size(1), ptr<float>(out), ptr<float>(ratio), stream_of(h)),
+        "xenc_hook_add");
+  return {out, ratio};
+}
+
+// One hooked layer of a decode step over one library, rows h [M, d_m]: hook_query, route_read (rows of one
+// library), hook_write and hook_add in one call, the same launches and bits.  maps = (A, gate_w, gate_b,
+// log_gain, B), pool = (S, pages, chunk_page, chunk_nvalid, chunk_ptr); sizes = (position of the layer in
+// gate_b / log_gain, top_k, cmax, kk, nsplit, workspace rows), scales = (eps, gain, route_temp, read_temp).
+// -> (h + delta, w [M, cmax], mean of |delta| / |h|).
+std::tuple<at::Tensor, at::Tensor, at::Tensor> hook_layer(const at::Tensor& h, at::TensorList maps,
+                                                          const c10::optional<at::Tensor>& a_bias,
+                                                          const c10::optional<at::Tensor>& b_bias, at::TensorList pool,
+                                                          c10::IntArrayRef sizes, c10::ArrayRef<double> scales,
+                                                          bool softmax, at::Tensor& workspace) {
+  TORCH_CHECK_VALUE(maps.size() == 5 && pool.size() == 5 && sizes.size() == 6 && scales.size() == 4,
+                    "hook_layer: 5 maps, 5 pool tensors, 6 sizes and 4 scales");
+  const c10::DeviceGuard guard(h.device());
+  auto [hn, q] = hook_query(h, maps[0], a_bias, scales[0]);
+  const at::Tensor group = at::zeros({h.size(0)}, i32(h));
+  auto [w, idx, wsel, r] = route_read(q, pool[0], pool[1], pool[2], pool[3], pool[4], group, sizes[1], scales[2], sizes[2],
+                                      sizes[3], scales[3], softmax, sizes[4], workspace, sizes[5]);
+  const int64_t p = sizes[0];
+  const at::Tensor delta = hook_write(hn, r, maps[1], maps[2].slice(0, p, p + 1), maps[3].slice(0, p, p + 1), scales[1],
+                                      maps[4], b_bias);
+  auto [out, ratio] = hook_add(h, delta);
+  return {out, w, ratio.mean()};
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(xenc, m) {
@@ -273,6 +343,12 @@ TORCH_LIBRARY_FRAGMENT(xenc, m) {
   m.def("paged_decode_joint(Tensor q, Tensor op_k, Tensor op_v, Tensor op_bt, Tensor op_len, Tensor own_k, "
         "Tensor own_v, Tensor own_bt, Tensor own_len, float scale, SymInt nsplit, SymInt chunk, "
         "Tensor(a!) workspace, SymInt max_n, Tensor(b!) out) -> ()");
+  m.def("hook_query(Tensor h, Tensor A, Tensor? bias, float eps) -> (Tensor, Tensor)");
+  m.def("hook_write(Tensor hn, Tensor r, Tensor gate_w, Tensor gate_b, Tensor log_gain, float gain_scale, Tensor W, "
+        "Tensor? bias) -> Tensor");
+  m.def("hook_add(Tensor h, Tensor delta) -> (Tensor, Tensor)");
+  m.def("hook_layer(Tensor h, Tensor[] maps, Tensor? a_bias, Tensor? b_bias, Tensor[] pool, int[] sizes, "
+        "float[] scales, bool softmax, Tensor(a!) workspace) -> (Tensor, Tensor, Tensor)");
   m.def("read_entries(Tensor q, Tensor w, Tensor? idx, Tensor frag_k_scores, Tensor frag_v_readout, Tensor chunk_ptr, "
         "Tensor row_ptr, Tensor chunk_page, Tensor chunk_nvalid, SymInt max_rows, SymInt tile_rows, SymInt blocks, "
         "SymInt slots, float read_temp, bool softmax) -> Tensor");
@@ -292,6 +368,10 @@ TORCH_LIBRARY_IMPL(xenc, CUDA, m) {
   m.impl("library_read", &library_read);
   m.impl("route_read", &route_read);
   m.impl("paged_decode_joint", &paged_decode_joint);
+  m.impl("hook_query", &hook_query);
+  m.impl("hook_write", &hook_write);
+  m.impl("hook_add", &hook_add);
+  m.impl("hook_layer", &hook_layer);
   m.impl("read_entries", &read_entries);
   m.impl("library_read_entries", &library_read_entries);
   m.impl("library_read_entries_bwd", &library_read_entries_bwd);

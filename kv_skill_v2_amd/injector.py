@@ -12,6 +12,9 @@ in three stages:
     update     delta = gain_scale * gain * gate * B(r), then the LayerSelector if set  (HIP on
                the decode path, torch with autograd)
 
+Without a gradient, a few rows' query and update and every row's residual add run as HIP operators
+(xenc::hook_query, hook_write, hook_add), and a decode step's whole layer as one (xenc::hook_layer).
+
 The read goes through torch.ops.xenc: few rows without autograd take the split-K decode
 operators (xenc::route_topk, xenc::library_read), many rows or autograd the MFMA operators
 (xenc::route_rows, xenc::library_prefill_fwd, both differentiable).  With a LayerSelector the
@@ -31,10 +34,11 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 
 from . import ops
 from .depth import KVSkill, decoder_layers, for_reader
-from .interface import ModelInterface, apply_map
+from .interface import _EPS, ModelInterface, apply_map
 from .library import PAGE_ALIGN, Library
 from .selector import rms_norm
 
@@ -89,6 +93,12 @@ def write_delta(itf, hn: torch.Tensor, r: torch.Tensor, li: int, gain_scale: flo
     if not fused:
         return gain_scale * itf_gain(itf, li, hn) * gcal * itf_gate(itf, hn, li) * itf_write(itf, r)
     p = itf._pos[li]
+    hn2, r2, gw, gb, lg = _rows_fp32(hn), _rows_fp32(r), itf.gate_w, itf.gate_b, itf.log_gain
+    if (hn2 is not None and r2 is not None and _plain(hn, r) and all(_dense_fp32(t, r) for t in (B.weight, gw, gb, lg))
+            and (B.bias is None or _dense_fp32(B.bias, r))):
+        out = torch.ops.xenc.hook_write(hn2, r2, gw, gb[p:p + 1], lg[p:p + 1], float(gain_scale) * float(gcal), B.weight,
+                                        B.bias)
+        return out.view(*r.shape[:-1], B.weight.shape[0])
     scale = ops.gate_scale(hn.reshape(rows, hn.shape[-1]).float().contiguous(), _here(itf.gate_w, r),
                            _here(itf.gate_b, r)[p:p + 1], _here(itf.log_gain, r)[p:p + 1],
                            float(gain_scale) * float(gcal))
@@ -96,6 +106,27 @@ def write_delta(itf, hn: torch.Tensor, r: torch.Tensor, li: int, gain_scale: flo
     out = ops.write_back(r.reshape(rows, r.shape[-1]).contiguous(), _here(B.weight, r).contiguous(), None,
                          bias, scale)
     return out.view(*r.shape[:-1], B.weight.shape[0])
+
+
+def _rows_fp32(t: torch.Tensor) -> torch.Tensor | None:
+    """t [..., d] as fp32 rows the HIP row kernels take (a view), or None when it is not that."""
+    if not t.is_cuda or t.dtype != torch.float32 or t.shape[-1] % 4 or t.shape[-1] == 0 or not t.is_contiguous() \
+            or t.data_ptr() % 16:
+        return None
+    return t.reshape(-1, t.shape[-1])
+
+
+def _plain(*tensors) -> bool:
+    """No gradient, forward-mode tangent or autocast reaches these: HIP operators without a derivative
+    may stand in for the torch ones."""
+    if torch.is_autocast_enabled() or forward_ad._current_level >= 0:
+        return False
+    return not torch.is_grad_enabled() or not any(t.requires_grad for t in tensors)
+
+
+def _dense_fp32(w: torch.Tensor, like: torch.Tensor) -> bool:
+    """A weight the row operators take where it is: fp32, row-major, 16-byte aligned, on like's device."""
+    return (w.device == like.device and w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
 def _by_entries(rows: int) -> bool:
@@ -118,10 +149,20 @@ class _AddUpdate:
             return output
         packed = isinstance(output, tuple)
         h = output[0] if packed else output
+        out = inj._whole_layer(h, self.li)
+        if out is not None:
+            return (out, *output[1:]) if packed else out
         delta = inj._branch(h, self.li).to(h.dtype)
         mask = inj._pos_mask(h)
         if mask is not None:
             delta = delta * mask
+        rows = _rows_fp32(h) if delta.shape == h.shape and _plain(h, delta) else None
+        drows = None if rows is None else _rows_fp32(delta)
+        if drows is not None and rows.shape[0]:
+            out, ratio = torch.ops.xenc.hook_add(rows, drows)
+            inj.mag_terms.append(ratio.mean())
+            out = out.view(h.shape)
+            return (out, *output[1:]) if packed else out
         ratio = torch.linalg.vector_norm(delta.float(), dim=-1) / (torch.linalg.vector_norm(h.float(), dim=-1) + 1e-6)
         inj.mag_terms.append(ratio.mean())
         out = h + delta
@@ -161,6 +202,10 @@ class SkillInjector:
     def _pos_mask(self, h: torch.Tensor):
         return None
 
+    def _whole_layer(self, h: torch.Tensor, li: int) -> torch.Tensor | None:
+        """The hooked layer's output in one operator, where there is one for it (else None)."""
+        return None
+
     def _attach(self) -> None:
         blocks = decoder_layers(self.model)
         self._handles.extend(blocks[li].register_forward_hook(_AddUpdate(self, li)) for li in self.itf.inject_layers)
@@ -177,8 +222,15 @@ class SkillInjector:
         self.mag_terms.clear()
 
     def _query(self, h: torch.Tensor):
+        itf, rows = self.itf, _rows_fp32(h)
+        A = itf.A if type(itf) is ModelInterface else None
+        if (rows is not None and isinstance(A, nn.Linear) and 0 < rows.shape[0] <= _FUSED_WRITE_ROWS
+                and _dense_fp32(A.weight, h) and (A.bias is None or _dense_fp32(A.bias, h))
+                and A.weight.shape[0] % 4 == 0 and not _needs_grad(itf, h) and _plain(h)):
+            hn, q = torch.ops.xenc.hook_query(rows, A.weight, A.bias, _EPS)
+            return hn.view(h.shape), q.view(*h.shape[:-1], -1)
         hn = rms_norm(h)
-        return hn, itf_query(self.itf, hn)
+        return hn, itf_query(itf, hn)
 
 
 class XEncInjector(SkillInjector):
@@ -366,6 +418,38 @@ class LibraryInjector(XEncInjector):
         if want_train:
             self.attn_terms.append(maps[1].float())
 
+    def _whole_layer(self, h: torch.Tensor, li: int) -> torch.Tensor | None:
+        """A decode step's layer (a few rows, no gradient, no selector, diagnostics or position mask) as one
+        operator, xenc::hook_layer: the launches and the bits of _branch and the residual add."""
+        if (torch.is_grad_enabled() or self.lib is None or self.selector is not None or self.force_attn is not None
+                or self.record_attn or any(getattr(getattr(self, name), "__func__", None) is not own
+                                           for name, own in _LAYER_PARTS)):
+            return None
+        itf, rows = self.itf, _rows_fp32(h)
+        if rows is None or not 0 < rows.shape[0] <= ops.DECODE_MAX_ROWS or type(itf) is not ModelInterface \
+                or not _plain(h):
+            return None
+        A, B, gw, gb, lg = itf.A, itf.B, itf.gate_w, itf.gate_b, itf.log_gain
+        if not (isinstance(A, nn.Linear) and isinstance(B, nn.Linear)):
+            return None
+        maps = [A.weight, gw, gb, lg, B.weight]
+        pool = self._pool(li, h)
+        if (pool.values is not None or pool.d != pool.d_valid or pool.d != A.weight.shape[0]
+                or rows.shape[1] != B.weight.shape[0]
+                or not all(_dense_fp32(t, h) for t in maps + [b for b in (A.bias, B.bias) if b is not None])):
+            return None
+        M, top_k = rows.shape[0], self.top_k
+        kk = pool.kept(top_k)
+        ns = ops.default_nsplit(M * kk, pool.slots_per_page)
+        ws, ws_rows = ops._WORKSPACES.get(rows.device, ops.stream_handle(rows.device), M, kk, ns, pool.d)
+        out, w, ratio = torch.ops.xenc.hook_layer(
+            rows, maps, A.bias, B.bias, [pool.S, pool.pages, pool.chunk_page, pool.chunk_nvalid, pool.chunk_ptr],
+            [itf._pos[li], top_k, pool.cmax, kk, ns, ws_rows],
+            [_EPS, self.gain_scale, self.route_temp, self.read_temp], self.read_softmax, ws)
+        self.last_route = w.view(*h.shape[:-1], -1)
+        self.mag_terms.append(ratio)
+        return out.view(h.shape)
+
     def _branch(self, h: torch.Tensor, li: int) -> torch.Tensor:
         if self.lib is None:                               # single-skill path
             delta = super()._branch(h, li)
@@ -390,6 +474,9 @@ class LibraryInjector(XEncInjector):
             delta = self.selector.apply(delta, h, li)
         return delta
 
+
+# The methods _whole_layer stands in for: a subclass or an instance that replaces one keeps the long way.
+_LAYER_PARTS = [(name, getattr(LibraryInjector, name)) for name in ("_branch", "_query", "_read", "_pool", "_pos_mask")]
 
 __all__ = ["SkillInjector", "XEncInjector", "LibraryInjector", "itf_query", "itf_gate", "itf_gain",
            "itf_write", "write_delta", "rms_norm", "apply_map"]

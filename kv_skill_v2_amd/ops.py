@@ -1229,6 +1229,9 @@ def branch_read(q: torch.Tensor, lib_: PagedLibrary, top_k: int = 0, read_temp: 
     tile = 0
     if by_entries and not grad and prefill_ok(lib_) and (M > DECODE_MAX_ROWS or lib_.values is not None):
         tile = _entry_tile([M], lib_, lib_.kept(int(top_k)))
+    if not grad and M <= DECODE_MAX_ROWS and lib_.values is None:   # routing and read as one operator, the same bits
+        w, _, _, r = route_read_decode(_pad_rows(q, lib_), lib_, None, top_k, route_temp, read_temp, read_softmax)
+        return (r[:, :lib_.d_valid] if lib_.d != lib_.d_valid else r), w
     w, idx, wsel = route_rows(q, lib_, top_k, route_temp)
     if tile:   # the pairs the routing kept
         r = _read_entries(_pad_rows(q, lib_), w, idx, lib_, tile, read_temp, read_softmax)

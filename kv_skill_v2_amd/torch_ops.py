@@ -378,6 +378,27 @@ def _routed_backward(ctx, dr, dw, _didx, _dwsel, _dp):
 library_read_routed.register_autograd(_routed_backward, setup_context=_routed_setup)
 
 
+# ----------------------------------------------------------------------------- a hooked layer around its read
+@torch.library.register_fake("xenc::hook_query")
+def _(h, A, bias, eps):
+    return h.new_empty(h.shape), h.new_empty(h.shape[0], A.shape[0])
+
+
+@torch.library.register_fake("xenc::hook_write")
+def _(hn, r, gate_w, gate_b, log_gain, gain_scale, W, bias):
+    return r.new_empty(r.shape[0], W.shape[0])
+
+
+@torch.library.register_fake("xenc::hook_add")
+def _(h, delta):
+    return h.new_empty(h.shape), h.new_empty(h.shape[0])
+
+
+@torch.library.register_fake("xenc::hook_layer")
+def _(h, maps, a_bias, b_bias, pool, sizes, scales, softmax, workspace):
+    return h.new_empty(h.shape), h.new_empty(h.shape[0], sizes[2]), h.new_empty(())
+
+
 # ----------------------------------------------------------------------------- the read by entries
 # (csrc/entries.hip; defined and implemented in csrc/torch_ops.cpp)
 @torch.library.register_fake("xenc::read_entries")
