@@ -14,10 +14,10 @@ of its own output buffer (callers clone it if they keep it across calls).  A cal
 nothing, reads no device value on the host and synchronises nothing, so it can be captured in a
 HIP graph and replayed with new lengths / block tables.  `block_n` is accepted for signature
 compatibility (it sized the reference's key tile); the HIP kernel picks its own tiling.  `chunk`
-(keys per split) keeps the reference's meaning and default (1024); chunk=None, an addition of this
-build, chooses it from max_n, hkv and max_keys for about 1024 workgroups at full capacity (faster
-at small batches: 37 against 48 us for one row over 16k keys).  The split only changes the order
-of the LSE merge, not what is computed.
+(the most keys per split) keeps the reference's default (1024); chunk=None, an addition of this
+build, chooses it from max_n, hkv and max_keys.  A reader whose splits would leave CUs idle reads each
+in halves, quarters, ... (`launch_splits`).  The split only changes the order of the LSE merge, not
+what is computed.
 """
 
 from __future__ import annotations
@@ -55,11 +55,12 @@ class DecodeReader:
         device = torch.device(device)
         if device.type != "cuda":
             raise DecodeReaderDeviceError("DecodeReader runs only on a ROCm GPU (there is no CPU path)")
-        if chunk is None:
+        auto = chunk is None
+        if auto:
             cus = torch.cuda.get_device_properties(device).multi_processor_count
             chunk = self.auto_chunk(max_n, hkv, max_keys, cus)
-        self.max_n, self.chunk, self.block_n = int(max_n), int(chunk), int(block_n)
-        self.S = max(1, math.ceil(max_keys / self.chunk))
+        self.max_n, self.block_n = int(max_n), int(block_n)
+        self.S, self.chunk = self.launch_splits(self.max_n, self.hkv, int(max_keys), int(chunk), 256 if auto else 800)
         L = lib()
         nbytes = L.xenc_joint_workspace_bytes(self.max_n, self.hkv, self.S, self.G, self.d)
         self.workspace = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
@@ -82,6 +83,24 @@ class DecodeReader:
         splits = max(1, int(cus) // units)
         chunk = max(512, -(-int(max_keys) // splits))
         return -(-chunk // 64) * 64
+
+    @staticmethod
+    def launch_splits(max_n: int, hkv: int, max_keys: int, chunk: int, blocks: int) -> tuple[int, int]:
+        """(splits, keys per split) of a launch: `chunk` halved while that keeps at most `blocks` workgroups
+        at full capacity, 36 splits a row (their merge is serial) and 128 keys a split.  A workgroup
+        streams at 25-30 GB/s, so too few of them bound the read.  Ragged rows, us at chunk 1024 / the
+        halving: 5 rows x hkv 8 x 128, 5,000 keys 32 / 20 (256); one row x 4 x 256, 16,384 keys 40 / 33
+        (512; 36 at 256, 65 splits); 3 rows x 2 x 256, 900 keys 44 / 18 (128); 24 rows x 2 x 256, 6,000
+        keys 87 / 62 (512; 65 at 256, 1,152 workgroups).  An automatic chunk already aims at a workgroup
+        per CU (blocks = 256): only short operators go below it (3 rows, 900 keys 30 / 18)."""
+        span = chunk
+        while span > 128:
+            half = -(-(span // 2) // 64) * 64
+            s = -(-max_keys // half)
+            if half >= span or half < 128 or s > 36 or s * max_n * hkv > blocks:
+                break
+            span = half
+        return max(1, math.ceil(max_keys / span)), span
 
     @staticmethod
     def _pool(k: torch.Tensor, v: torch.Tensor, name: str):

@@ -198,3 +198,14 @@ def test_decode_reader_zero_rows(dev):
     args[0] = args[0][:0]
     out = dec(*args, 0.1)
     assert out.shape == (0, 8, 64)
+
+
+@pytest.mark.parametrize("max_n,hkv,max_keys,chunk,blocks,want", [
+    (5, 8, 5077, 1024, 800, (20, 256)), (1, 4, 16461, 1024, 800, (33, 512)), (32, 4, 16448, 1024, 800, (17, 1024)),
+    (3, 2, 977, 1024, 800, (8, 128)), (32, 4, 16448, 8256, 256, (2, 8256)), (4, 4, 100, 64, 800, (2, 64)),
+    (1, 1, 900, 1000, 800, (8, 128)), (1, 1, 1, 1024, 800, (1, 128))])
+def test_launch_splits(dev, max_n, hkv, max_keys, chunk, blocks, want):
+    """The launch's splits: every key covered, the caller's chunk never exceeded."""
+    say("op B splits", dict(max_n=max_n, hkv=hkv, max_keys=max_keys, chunk=chunk))
+    s, span = DecodeReader.launch_splits(max_n, hkv, max_keys, chunk, blocks)
+    assert (s, span) == want and s * span >= max_keys and span <= chunk
