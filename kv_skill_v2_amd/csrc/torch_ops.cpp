@@ -9,8 +9,9 @@
 //   xenc::library_read        the read of LibraryInjector._branch (xenc/injector.py:236-265)
 //   xenc::route_read          both in one call (the top-k inside the read kernel when it can)
 //   xenc::read_entries        the read of many rows by their routed (row, chunk) pairs, no gradient
-//   xenc::library_read_entries, library_read_entries_bwd   routing + that read, and its dQ (autograd
-//                             registered in torch_ops.py)
+//   xenc::library_read_entries, library_read_entries_bwd   routing + that read, and its dQ: its
+//                             autograd is here too (registered from Python, a call with this many
+//                             arguments spent 95 us of a small training step on its schema)
 //   xenc::hook_query, hook_write, hook_add   a hooked layer's query, update and residual add around
 //                             the read, for steps without a gradient
 //   xenc::hook_layer          a whole hooked layer of a decode step: the above and route_read
@@ -18,6 +19,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
 
 #include <algorithm>
@@ -241,6 +243,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tenso
   return {r, w, idx, wsel, p, list, count};
 }
 
+using EntriesOut = std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor>;
+
 at::Tensor library_read_entries_bwd(const at::Tensor& g, const at::Tensor& w, const at::Tensor& idx,
                                     const at::Tensor& p, const c10::optional<at::Tensor>& dw_ext, const at::Tensor& S,
                                     const at::Tensor& list, const at::Tensor& count, const at::Tensor& frag_v_scores,
@@ -260,6 +264,90 @@ at::Tensor library_read_entries_bwd(const at::Tensor& g, const at::Tensor& w, co
   E.scores(softmax ? 1 : 3, rows_f16(g, st), frag_v_scores, read_temp, &w, p, &ds, &gamma);
   return E.readout(ds, frag_k_readout, nullptr, ptr<const int>(idx), &w, &gamma, dw_ext ? &*dw_ext : nullptr, &S,
                    route_temp);
+}
+
+// Autograd of library_read_entries.  Both directions go through the dispatcher (fake tensors and
+// functionalisation see the two operators); no gradient is materialised for the outputs nothing
+// differentiates.
+class EntriesRead : public torch::autograd::Function<EntriesRead> {
+ public:
+  static torch::autograd::variable_list forward(
+      torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& S, const at::Tensor& chunk_ptr,
+      const at::Tensor& row_ptr, const at::Tensor& logit_tiles, const at::Tensor& route_tiles, c10::SymInt n_logit,
+      c10::SymInt n_route, c10::SymInt top_k, double route_temp, c10::SymInt cmax, c10::SymInt kk,
+      const at::Tensor& frag_k_scores, const at::Tensor& frag_v_readout, const at::Tensor& frag_v_scores,
+      const at::Tensor& frag_k_readout, const at::Tensor& chunk_page, const at::Tensor& chunk_nvalid,
+      c10::SymInt max_rows, c10::SymInt tile_rows, c10::SymInt slots, double read_temp, bool softmax) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    static const auto op = c10::Dispatcher::singleton()
+                               .findSchemaOrThrow("xenc::library_read_entries", "")
+                               .typed<decltype(library_read_entries)>();
+    auto [r, w, idx, wsel, p, list, count] =
+        op.call(q, S, chunk_ptr, row_ptr, logit_tiles, route_tiles, n_logit, n_route, top_k, route_temp, cmax, kk,
+                frag_k_scores, frag_v_readout, frag_v_scores, frag_k_readout, chunk_page, chunk_nvalid, max_rows,
+                tile_rows, slots, read_temp, softmax);
+    ctx->save_for_backward({w, idx, p, list, count, frag_v_scores, frag_k_readout, chunk_ptr, chunk_page, chunk_nvalid,
+                            row_ptr, S, route_tiles});
+    ctx->saved_data["n_route"] = n_route;
+    ctx->saved_data["max_rows"] = max_rows;
+    ctx->saved_data["tile_rows"] = tile_rows;
+    ctx->saved_data["slots"] = slots;
+    ctx->saved_data["d"] = q.sym_size(1);
+    ctx->saved_data["read_temp"] = read_temp;
+    ctx->saved_data["route_temp"] = route_temp;
+    ctx->saved_data["softmax"] = softmax;
+    ctx->mark_non_differentiable({idx, wsel, p, list, count});
+    ctx->set_materialize_grads(false);
+    return {r, w, idx, wsel, p, list, count};
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto v = ctx->get_saved_variables();
+    const at::Tensor &w = v[0], &idx = v[1], &p = v[2], &list = v[3], &count = v[4], &fvs = v[5], &fkr = v[6],
+                     &chunk_ptr = v[7], &chunk_page = v[8], &chunk_nvalid = v[9], &row_ptr = v[10], &S = v[11],
+                     &route_tiles = v[12];
+    auto& sd = ctx->saved_data;
+    const at::Tensor &dr = grads[0], &dw = grads[1];
+    const double route_temp = sd["route_temp"].toDouble();
+    c10::optional<at::Tensor> dwc;
+    if (dw.defined()) dwc = dw.contiguous();
+    at::Tensor dq;
+    if (dr.defined()) {
+      static const auto op = c10::Dispatcher::singleton()
+                                 .findSchemaOrThrow("xenc::library_read_entries_bwd", "")
+                                 .typed<decltype(library_read_entries_bwd)>();
+      dq = op.call(dr.contiguous(), w, idx, p, dwc, S, list, count, fvs, fkr, chunk_ptr, chunk_page, chunk_nvalid,
+                   row_ptr, sd["max_rows"].toSymInt(), sd["tile_rows"].toSymInt(), sd["slots"].toSymInt(),
+                   sd["read_temp"].toDouble(), sd["softmax"].toBool(), route_temp);
+    } else {   // only w reaches the loss: the routing term alone (nothing at all: 0)
+      dq = at::zeros_symint({w.sym_size(0), sd["d"].toSymInt()}, w.options());
+      if (dwc) {
+        static const auto op = c10::Dispatcher::singleton()
+                                   .findSchemaOrThrow("xenc::route_backward_", "")
+                                   .typed<void(at::Tensor&, const at::Tensor&, const at::Tensor&,
+                                               const c10::optional<at::Tensor>&, const at::Tensor&, const at::Tensor&,
+                                               const at::Tensor&, const at::Tensor&, c10::SymInt, double)>();
+        op.call(dq, w, at::zeros_like(w), dwc, S, chunk_ptr, row_ptr, route_tiles, sd["n_route"].toSymInt(), route_temp);
+      }
+    }
+    torch::autograd::variable_list out(23);
+    out[0] = dq;
+    return out;
+  }
+};
+
+EntriesOut library_read_entries_autograd(
+    const at::Tensor& q, const at::Tensor& S, const at::Tensor& chunk_ptr, const at::Tensor& row_ptr,
+    const at::Tensor& logit_tiles, const at::Tensor& route_tiles, c10::SymInt n_logit, c10::SymInt n_route,
+    c10::SymInt top_k, double route_temp, c10::SymInt cmax, c10::SymInt kk, const at::Tensor& frag_k_scores,
+    const at::Tensor& frag_v_readout, const at::Tensor& frag_v_scores, const at::Tensor& frag_k_readout,
+    const at::Tensor& chunk_page, const at::Tensor& chunk_nvalid, c10::SymInt max_rows, c10::SymInt tile_rows,
+    c10::SymInt slots, double read_temp, bool softmax) {
+  auto o = EntriesRead::apply(q, S, chunk_ptr, row_ptr, logit_tiles, route_tiles, n_logit, n_route, top_k, route_temp,
+                              cmax, kk, frag_k_scores, frag_v_readout, frag_v_scores, frag_k_readout, chunk_page,
+                              chunk_nvalid, max_rows, tile_rows, slots, read_temp, softmax);
+  return {o[0], o[1], o[2], o[3], o[4], o[5], o[6]};
 }
 
 // ---- a hooked layer around its read (xenc/injector.py:54-77, 185-197)
@@ -362,6 +450,8 @@ TORCH_LIBRARY_FRAGMENT(xenc, m) {
         "Tensor chunk_nvalid, Tensor row_ptr, SymInt max_rows, SymInt tile_rows, SymInt slots, float read_temp, "
         "bool softmax, float route_temp) -> Tensor");
 }
+
+TORCH_LIBRARY_IMPL(xenc, Autograd, m) { m.impl("library_read_entries", &library_read_entries_autograd); }
 
 TORCH_LIBRARY_IMPL(xenc, CUDA, m) {
   m.impl("route_topk", &route_topk);

@@ -423,33 +423,6 @@ def _(g, w, idx, p, dw_ext, S, list, count, frag_v_scores, frag_k_readout, chunk
     return g.new_empty(g.shape)
 
 
-def _entries_setup(ctx, inputs, output):
-    (q, S, chunk_ptr, row_ptr, _lt, route_tiles, _nl, n_route, _tk, route_temp, _cmax, _kk, _fks, _fvr, fvs, fkr,
-     chunk_page, chunk_nvalid, max_rows, tile_rows, slots, read_temp, softmax) = inputs
-    _, w, idx, _, p, lst, count = output
-    ctx.save_for_backward(w, idx, p, lst, count, fvs, fkr, chunk_ptr, chunk_page, chunk_nvalid, row_ptr, S, route_tiles)
-    ctx.sizes = (max_rows, tile_rows, slots, read_temp, softmax)
-    ctx.route = (n_route, route_temp)
-    ctx.d = q.shape[1]
-    ctx.mark_non_differentiable(*output[2:])
-    ctx.set_materialize_grads(False)   # (else every backward fills zeros for p, idx and w_sel)
-
-
-def _entries_backward(ctx, dr, dw, *_):
-    w, idx, p, lst, count, fvs, fkr, chunk_ptr, chunk_page, chunk_nvalid, row_ptr, S, route_tiles = ctx.saved_tensors
-    dw = None if dw is None else dw.contiguous()
-    if dr is None:  # only w reaches the loss: the routing term alone
-        dq = torch.zeros(w.shape[0], ctx.d, dtype=torch.float32, device=w.device)
-        torch.ops.xenc.route_backward_(dq, w, torch.zeros_like(w), dw, S, chunk_ptr, row_ptr, route_tiles, *ctx.route)
-    else:
-        dq = torch.ops.xenc.library_read_entries_bwd(dr.contiguous(), w, idx, p, dw, S, lst, count, fvs, fkr, chunk_ptr,
-                                                     chunk_page, chunk_nvalid, row_ptr, *ctx.sizes, ctx.route[1])
-    return (dq,) + (None,) * 22
-
-
-torch.library.register_autograd("xenc::library_read_entries", _entries_backward, setup_context=_entries_setup)
-
-
 # ----------------------------------------------------------------------------- op B
 _JOINT_DTYPES = {torch.float16: 0, torch.bfloat16: 1}
 

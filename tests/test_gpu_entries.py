@@ -129,3 +129,52 @@ def test_entries_rule(dev):
     assert ops._entry_tile_of(48, 3, 333 * 4, 16, 16, 4, 512, 2048) == 32
     assert ops._entry_tile_of(1024, 16, 2048 * 8, 64, 64, 8, 512, 2048) == 64
     assert ops._entry_tile_of(2048, 64, 8192 * 32, 128, 32, 32, 512, 2048) == 0
+
+
+CHECKS = ("test_schema", "test_autograd_registration", "test_faketensor", "test_aot_dispatch_dynamic")
+
+
+def test_entries_operators(dev, monkeypatch):
+    """opcheck (schema, fakes, autograd, AOT dispatch with the backward) of the operators; saved tensors
+    packed and unpacked by hooks; a gradient of the gradient-free outputs; no gradient at all."""
+    say("entries operators")
+    P = synth.pool([4, 3], 128, 128, device="cpu", tail_lo=1)
+    lib = ops.PagedLibrary(*(t.to(dev) for t in (P.pages, P.chunk_page, P.chunk_nvalid, P.chunk_ptr, P.S)),
+                           n_chunks=P.n_chunks, nvalid=P.nvalid)
+    plan = lib.plan([70, 66])
+    q = synth.queries(plan.M, lib.d, device=dev, seed=4).requires_grad_(True)
+    fk, fv, fvs, fkr, chunk_ptr, chunk_page, chunk_nvalid, row_ptr, *_ = ops._prefill_operands(lib, plan)
+    args = (q, lib.S, chunk_ptr, row_ptr, plan.logit_tiles, plan.route_tiles, plan.n_logit, plan.n_route, 2, 10.0,
+            lib.cmax, 2, fk, fv, fvs, fkr, chunk_page, chunk_nvalid, 70, 32, 128, 12.0, True)
+    # (a list's tail past its chunk's count is never written, so whole outputs are not compared here)
+    torch.library.opcheck(torch.ops.xenc.library_read_entries.default, args, test_utils=CHECKS[:3])
+    r, w, idx, _, p, lst, count = torch.ops.xenc.library_read_entries(*args)
+    assert r.requires_grad and w.requires_grad and not any(t.requires_grad for t in (idx, p, lst, count))
+    g = torch.randn(r.shape, device=dev, generator=torch.Generator(device=dev).manual_seed(1))
+    want, = torch.autograd.grad(r, q, g, retain_graph=True)
+    from functorch.compile import aot_function, nop
+    traced = aot_function(lambda *a: torch.ops.xenc.library_read_entries(*a)[:2], nop, nop)
+    rt, wt = traced(*args)
+    got, = torch.autograd.grad(rt, q, g)
+    assert torch.equal(rt, r) and torch.equal(wt, w) and torch.equal(got, want)
+    bargs = (g, w.detach(), idx, p, torch.randn_like(w), lib.S, lst, count, fvs, fkr, chunk_ptr, chunk_page, chunk_nvalid,
+             row_ptr, 70, 32, 128, 12.0, True, 10.0)
+    torch.library.opcheck(torch.ops.xenc.library_read_entries_bwd.default, bargs,
+                          test_utils=("test_schema", "test_faketensor"))
+    for i, blocks in ((None, 1), (idx, 1)):
+        rargs = (q.detach(), w.detach(), i, fk, fv, chunk_ptr, row_ptr, chunk_page, chunk_nvalid, 70, 32, blocks, 128, 12.0,
+                 True)
+        torch.library.opcheck(torch.ops.xenc.read_entries.default, rargs, test_utils=CHECKS)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(1) or t.cpu(), lambda t: t.to(dev)):
+        r2 = torch.ops.xenc.library_read_entries(*args)[0]
+        got, = torch.autograd.grad(r2, q, g)
+    assert len(packed) == 13 and torch.equal(got, want)
+    monkeypatch.setattr(ops, "_entry_tile", lambda *a: 32)
+    with torch.no_grad():
+        r3, w3 = ops.library_read(q, lib, plan, top_k=2)
+    assert torch.equal(r3, r.detach()) and not r3.requires_grad and torch.equal(w3, w.detach())
+    with torch.inference_mode():
+        assert torch.equal(ops.library_read(q.detach().clone(), lib, plan, top_k=2)[0], r3)
+    dq, = torch.autograd.grad(w.sum() * 0.0 + r.sum() * 0.0, q)
+    assert float(dq.abs().max()) == 0.0
