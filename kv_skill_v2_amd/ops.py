@@ -944,7 +944,7 @@ def library_read(q: torch.Tensor, lib_: PagedLibrary, plan: RowPlan, top_k: int 
         # The routed (row, chunk) pairs only; reading every chunk without a gradient stays equal, bit for
         # bit, to route_topk_rows and prefill_forward.
         grad = torch.is_grad_enabled() and q.requires_grad
-        tile = _entry_tile(plan.rows, lib_, kk) if grad or kk < lib_.cmax else 0
+        tile = _entry_tile(plan.rows, lib_, kk, grad) if grad or kk < lib_.cmax else 0
         if tile:
             return torch.ops.xenc.library_read_entries(
                 q, lib_.S, chunk_ptr, row_ptr, plan.logit_tiles, plan.route_tiles, plan.n_logit, plan.n_route,
@@ -1107,32 +1107,37 @@ def prefill_ok(lib_: PagedLibrary) -> bool:
     return lib_.d % 64 == 0 and lib_.slots_per_page % 64 == 0 and lib_.slots_per_page <= 512
 
 
-def _entry_tile(rows: list[int], lib_: PagedLibrary, kk: int) -> int:
+def _entry_tile(rows: list[int], lib_: PagedLibrary, kk: int, grad: bool = False) -> int:
     """0: read every row against every chunk in 128-row tiles (csrc/prefill.hip); 32 or 64: read the
     kept (row, chunk) pairs grouped by chunk, that many per workgroup (csrc/entries.hip)."""
     pairs = list(zip(rows, lib_.n_chunks))
     return _entry_tile_of(sum(-(-m // 128) * c for m, c in pairs), sum(-(-m // 128) for m in rows),
                           sum(m * min(c, kk) for m, c in pairs), sum(lib_.n_chunks), lib_.cmax, kk,
-                          lib_.slots_per_page, lib_.d)
+                          lib_.slots_per_page, lib_.d, grad)
 
 
 @lru_cache(maxsize=1024)
-def _entry_tile_of(tiles: int, row_tiles: int, entries: int, n_chunks: int, cmax: int, kk: int, N: int, d: int) -> int:
+def _entry_tile_of(tiles: int, row_tiles: int, entries: int, n_chunks: int, cmax: int, kk: int, N: int, d: int,
+                   grad: bool = False) -> int:
     """The cheaper by this model, in us, fitted to measured forward kernels (the backward repeats the
     same two products, so the order holds for it).  Dense: a scores round of 256 workgroups 48 (a
-    full one 65), a readout k step 1.05, both at d = 2048.  Entries: a scores round 31 (32 rows) or 42
-    (64), a readout workgroup's 22 or 42 ns of the GPU, the partials' read at 6 TB/s, lists and launches.
-    Measured per call, dense against entries: 333 rows, top-4 of 16 chunks of 512 x 2048 208 / 57
+    full one 65), a readout k step 1.05, both at d = 2048.  Entries: scores 31 up to 150 tiles of 32
+    rows (then by their pages' share of the L2s), 42 a round of 256 tiles of 64, a readout
+    workgroup's 22 or 42 ns of the GPU, the partials' read at 6 TB/s, lists and launches.  Measured per call, dense against entries: 333 rows, top-4 of 16 chunks of 512 x 2048 208 / 57
     us; 1000 rows, top-8 and all of 16: 218 / 126 and 218 / 177; 2048 rows, top-8 of 64: 858 / 308;
-    2048 rows, top-4 of 8: 176 / 140; a training step of 4 x 2048 rows, top-4 of 32: 2.22 / 1.04 ms."""
+    2048 rows, top-4 of 8: 176 / 140; a training step of 4 x 2048 rows, top-4 of 32: 2.22 / 1.04 ms.
+    With a gradient a dense call takes the host 150 us whatever its kernels do (the Python side of its
+    operators: a step of 2 x 343 rows, all of 3-4 chunks of 128 x 320, 257 dense / 73 by entries; 4 x 734
+    rows, all of 7-14 of 256 x 320, 252 / 147), so below that the entries' own time decides."""
     D = d / 2048
     dense = max(48, 65 * tiles / 256) * D + 1.05 * cmax * (N / 64) * max(1, row_tiles * -(-d // 256) / 256)
-    best, tile = dense, 0
+    best, tile = max(dense, 150.0) if grad else dense, 0
     for rt, scores, out in ((32, 31, 0.022), (64, 42, 0.042)):
         if rt == 64 and N <= 128:
             continue
         t = entries / rt + (n_chunks / 2 if kk < cmax else 0)   # (a chunk's last tile is half full on average)
-        cost = scores * D * max(N, 128) / 512 * max(1, math.ceil(t / 256)) + 8 + t * -(-d // 256) * out * N / 512 + 6
+        rounds = max(1, t / 150 if rt == 32 else math.ceil(t / 256))
+        cost = scores * D * max(N, 128) / 512 * rounds + 8 + t * -(-d // 256) * out * N / 512 + 6
         if kk > 1:
             cost += entries * d * 4 / 6e6 + 3
         if cost < best:
