@@ -382,7 +382,15 @@ __global__ __launch_bounds__(kRouteThreads) void route_rows_logits_kernel(
 }
 
 constexpr int kSelectWaves = 4;
-constexpr int kSplitRouteRows = 256;   // below this many rows xenc_route_topk splits rows over waves
+// xenc_route_topk takes one wave per (row, two chunks) and a wave per row's top-k for fewer than 256 rows
+// (a workgroup per row leaves CUs idle), and again for many long rows, where a workgroup per row
+// streams its row with one dot's loads in flight.  us per call, workgroup per row / split, d = 2048:
+// 256 rows x 16 chunks 6.0 / 8.1, 1000 x 4 12.3 / 8.1, 1000 x 16 17.9 / 10.8, 2048 x 16 31 / 16, 512 x
+// 64 15.3 / 17.4, 2048 x 64 54 / 50, 8192 x 64 304 / 190; d = 256: 256 x 16 5.5 / 8.2, 8192 x 16 22 / 13.
+// The same dots and selection: the same bits.
+bool split_route(int M, int d, int chunks) {
+  return M < 256 || (long long)M * d >= (chunks <= 16 ? 1LL << 20 : 1LL << 22);
+}
 
 // Library of row m: q_group[m] (clamped) when given, else the g with row_ptr[g] <= m < row_ptr[g+1].
 __global__ __launch_bounds__(kSelectWaves * kWave) void route_rows_select_kernel(
@@ -497,9 +505,8 @@ extern "C" int xenc_route_topk(const float* q, long long ldq, int M, int d, cons
   constexpr int NW = 8;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int cb4 = (d + 255) / 256;
-  // Fewer rows than about one per CU: one wave per (row, chunk), then the wave top-k per row.
   const size_t sel_lds = (size_t)kSelectWaves * 3 * select_lds_stride((int)ldw) * sizeof(float);
-  if (M < kSplitRouteRows && sel_lds <= 64 * 1024) {
+  if (split_route(M, d, ldw) && sel_lds <= 64 * 1024) {
     const int rc = launch_route_dots(q, ldq, M, d, S, chunk_ptr, q_group, G, w_dense, (int)ldw, st);
     if (rc != XENC_OK) return rc;
     hipLaunchKernelGGL(route_rows_select_kernel, dim3((M + kSelectWaves - 1) / kSelectWaves),

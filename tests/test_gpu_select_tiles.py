@@ -76,3 +76,17 @@ def test_row_plan_tables(dev, n_lib):
         t = getattr(plan, name)
         assert t.is_cuda and t.dtype == torch.int32
         assert t.cpu().tolist() == [sum(per[:i]) for i in range(n_lib + 1)], name
+
+
+@pytest.mark.parametrize("M,C,d", [(300, 9, 2048), (512, 5, 2048), (513, 33, 2048), (1030, 16, 1024), (2050, 40, 2048)])
+def test_route_topk_is_one_result(dev, M, C, d):
+    """Routing with a workgroup per row and split over waves: either side of the line the same bits as calls
+    of fewer than 256 rows."""
+    say("route topk rows", dict(M=M, C=C, d=d))
+    P = synth.pool([C], 64, d, device="cpu")
+    lib = ops.PagedLibrary(*(t.to(dev) for t in (P.pages, P.chunk_page, P.chunk_nvalid, P.chunk_ptr, P.S)),
+                           n_chunks=P.n_chunks, nvalid=P.nvalid)
+    q = synth.queries(M, d, device=dev, seed=8)
+    got = ops.route_topk(q, lib, None, 3)
+    want = [torch.cat(t) for t in zip(*(ops.route_topk(x, lib, None, 3) for x in q.split(200)))]
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
