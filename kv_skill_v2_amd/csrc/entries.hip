@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kListThreads) void entries_list_kernel(const int* _
 // readout (MODE 4): p = 2^(s - m) with m the block's max rounded up to a whole number, and stats
 // [entry][block] = (m, sum of the block's p), so the blocks join by exact powers of two.
 // 333 rows, top-4 of 16 chunks of 512 x 2048: 48 us (128-row tiles over all pairs), 31 us whole
-// chunks, 13 us in 4 blocks.
+// chunks, 16 us in 4 blocks.
 template <int MODE, int SG, int NT>
 __global__ __launch_bounds__(kEntThreads) void entries_scores_kernel(
     const EntryArgs A, const _Float16* __restrict__ X, float temp, _Float16* __restrict__ P,
