@@ -359,15 +359,14 @@ def route_topk(q: torch.Tensor, lib_: PagedLibrary, q_group=None, top_k: int = 0
 
 
 def default_nsplit(units: int, slots_per_page: int) -> int:
-    """Slot splits per routed page.  With >= 256 (query, page) units one workgroup per page
+    """Slot splits per routed page.  With >= 128 (query, page) units one workgroup per page
     (measured best on the B = 64 batched decode); fewer units are split so that about
-    min(8 * units, 256) workgroups stream the pages, in pieces of >= 32 slots.  Very few units
-    stay at 8 splits per page: one query x 4 pages (the single-sequence decode) measured 34.4 / 23.4
-    / 18.9 / 17.8 / 20.0 / 26.9 us per step at 1 / 2 / 4 / 8 / 16 / 32 splits, 16 units 27 / 23.0 /
-    23.2 at 4 / 8 / 16.  Pages of 512 x 2048, at min(8 * units, 128) workgroups and here: 24 units 20.5
-    / 19.0 us (6 and 8 splits), 64 units 37 / 33.5 (2 and 4), 128 units 62 / 53 (1 and 2)."""
+    min(8 * units, 128) workgroups stream the pages, in pieces of >= 32 slots.  Very few units
+    stay at 8 splits per page because the last workgroup merges every partial: one query x 4
+    pages (the single-sequence decode) measured 34.4 / 23.4 / 18.9 / 17.8 / 20.0 / 26.9 us per
+    step at 1 / 2 / 4 / 8 / 16 / 32 splits."""
     units = max(units, 1)
-    want = max(1, math.ceil(min(8 * units, 256) / units))
+    want = max(1, math.ceil(min(8 * units, 128) / units))
     return int(max(1, min(want, max(1, slots_per_page // 32), 64)))
 
 
